@@ -14,6 +14,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include "bottom_kernels.h"
 #include "box_kernels.h"
 #include "nodal_kernels.h"
 
@@ -91,6 +92,37 @@ __device__ inline double eb_apply_node(const EBLev& L, const double* x, const do
     diag = dg;
     return acc;
 }
+
+// The rows of the EB operator for the bottom solve: inactive nodes are held at zero.
+struct EBRows {
+    static constexpr int NS = 27;
+    static constexpr bool kRedBlack = false;
+    EBLev L;
+    __device__ int dim(int d) const { return L.g.nn[d]; }
+    __device__ int per(int d) const { return L.g.per[d]; }
+    __device__ bool row(int id, int i, int j, int k, double (&C)[NS]) const {
+        const KGeom& g = L.g;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) C[s] = 0.0;
+#pragma unroll
+        for (int a = 0; a < 8; ++a) {
+            const int ax = a & 1, ay = (a >> 1) & 1, az = a >> 2;
+            const int c0 = eb_cell(g, 0, i, ax), c1 = eb_cell(g, 1, j, ay), c2 = eb_cell(g, 2, k, az);
+            if (c0 < 0 || c1 < 0 || c2 < 0) continue;
+            const int ci = L.cidx[c0 + (long)g.n[0] * (c1 + (long)g.n[1] * c2)];
+            if (ci == -2) continue;
+            const double* K = ci >= 0 ? L.K + 64L * ci : L.E;
+            const double w = ci >= 0 ? 1.0
+                                     : L.sig[(c0 + 1) + (long)g.sg[0] * ((c1 + 1) + (long)g.sg[1] * (c2 + 1))];
+            const int p = (1 - ax) | ((1 - ay) << 1) | ((1 - az) << 2);
+#pragma unroll
+            for (int m = 0; m < 8; ++m)
+                C[(ax + (m & 1)) + 3 * (ay + ((m >> 1) & 1)) + 9 * (az + (m >> 2))] -= w * K[p * 8 + m];
+        }
+        return L.mask[id] != 0;
+    }
+};
+MGX_BOTTOM_INSTANCE(extern, EBRows, double);
 
 static __global__ void __launch_bounds__(256) eb_stencil_kernel(EBArgs a, int mode) {
     int i, j, k;

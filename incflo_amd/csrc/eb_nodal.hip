@@ -6,6 +6,7 @@
 #include <cmath>
 #include <cstring>
 
+#include "bottom_kernels.h"
 #include "eb_nodal.h"
 #include "mgx_ctx.h"
 
@@ -322,61 +323,6 @@ __global__ void eb_subtract_masked_kernel(const unsigned char* __restrict__ mask
     if (id < n && mask[id]) a[id] -= s[0];
 }
 
-// one-workgroup BiCGStab (van der Vorst 1992) on the coarsest EB level, FP64,
-// vectors in global memory; inactive nodes hold 0; mean removed when singular
-// The EB nodal operator in FP64 for the bottom solve: inactive nodes are held
-// at zero and the singular mean is over the active ones; its smoother is the
-// V-cycle's weighted Jacobi sweep.
-struct EBBottomOp {
-    EBLev L;
-    double nact;
-    double omega;
-    __device__ long size() const { return (long)L.g.nn[0] * L.g.nn[1] * L.g.nn[2]; }
-    __device__ bool held(long id) const { return !L.mask[id]; }
-    __device__ double nfree() const { return nact; }
-    __device__ void node(long id, int& i, int& j, int& k) const {
-        i = (int)(id % L.g.nn[0]);
-        j = (int)((id / L.g.nn[0]) % L.g.nn[1]);
-        k = (int)(id / ((long)L.g.nn[0] * L.g.nn[1]));
-    }
-    __device__ void apply(const double* in, double* out, long n) const {
-        __syncthreads();
-        for (long id = threadIdx.x; id < n; id += blockDim.x) {
-            int i, j, k;
-            node(id, i, j, k);
-            double dg;
-            out[id] = L.mask[id] ? eb_apply_node(L, in, nullptr, i, j, k, dg) : 0.0;
-        }
-        __syncthreads();
-    }
-    __device__ void smooth(const BottomVecs& V, long n) const {
-        __syncthreads();
-        for (long id = threadIdx.x; id < n; id += blockDim.x) {
-            int i, j, k;
-            node(id, i, j, k);
-            double u = 0.0;
-            if (L.mask[id]) {
-                double dg;
-                const double lx = eb_apply_node(L, V.x, nullptr, i, j, k, dg);
-                if (dg != 0.0) u = V.x[id] + omega * (V.b[id] - lx) / dg;
-            }
-            V.t[id] = u;
-        }
-        __syncthreads();
-        for (long id = threadIdx.x; id < n; id += blockDim.x) V.x[id] = V.t[id];
-        __syncthreads();
-    }
-};
-
-__global__ void __launch_bounds__(1024) eb_bottom_kernel(EBLev L, const double* __restrict__ b_in,
-                                                         double* __restrict__ x_out, double* work,
-                                                         int kind, int maxiter, double rtol,
-                                                         double omega, int singular, double nact) {
-    __shared__ double red[16];
-    const EBBottomOp op{L, nact, omega};
-    bottom_solve_body(op, b_in, x_out, work, kind, maxiter, rtol, singular, nullptr, red);
-}
-
 void node_mask(const NodalGeom& g, const std::vector<int>& cidx, std::vector<unsigned char>& m) {
     m.assign(g.nnode(), 0);
     for (int k = 0; k < g.nn[2]; ++k)
@@ -483,7 +429,8 @@ void EBNodal::setup(const NodalGeom& g0, int nlev, const std::vector<int>& type,
         MGX_HIP(hipMemset(lv.x_buf.p, 0, nn * sizeof(double)));
         MGX_HIP(hipMemset(lv.x2_buf.p, 0, nn * sizeof(double)));
     }
-    bottom_work.alloc(7 * L.back().g.nnode() * sizeof(double));
+    bottom_work.alloc(bottom_work_doubles(L.back().g.nnode(), 27) * sizeof(double));
+    bottom_prepare<EBRows, double>();
     ready = true;
 }
 
@@ -555,14 +502,15 @@ void EBNodal::vcycle(const MGOpts& o, hipStream_t s) {
     }
     {
         EBLevelData& lb = L[nl - 1];
-        long nact = 0;
-        for (unsigned char m : lb.mask_h) nact += m;
-        const long nb = lb.g.nnode();
-        const int threads = nb >= 1024 ? 1024 : (nb >= 256 ? 256 : 64);
-        eb_bottom_kernel<<<1, threads, 0, s>>>(lev(nl - 1), lb.b_buf.as<double>(), lb.x_buf.as<double>(),
-                                               bottom_work.as<double>(), o.bottom_solver,
-                                               o.bottom_maxiter, o.bottom_rtol, nodal_omega(lb.g, o.omega),
-                                               lb.g.singular() ? 1 : 0, (double)nact);
+        BottomArgs ba{};
+        ba.work = bottom_work.as<double>();
+        ba.kind = o.bottom_solver;
+        ba.maxiter = o.bottom_maxiter;
+        ba.rtol = o.bottom_rtol;
+        ba.omega = nodal_omega(lb.g, o.omega);
+        ba.singular = lb.g.singular() ? 1 : 0;
+        bottom_launch<EBRows, double>(EBRows{lev(nl - 1)}, lb.g.nnode(), lb.b_buf.as<double>(),
+                                      lb.x_buf.as<double>(), ba, s);
     }
     for (int l = nl - 2; l >= 0; --l) {
         EBLevelData& lv = L[l];

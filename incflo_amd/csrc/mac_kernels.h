@@ -18,6 +18,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include "bottom_kernels.h"
 #include "nodal_kernels.h"
 
 namespace mgx {
@@ -350,72 +351,41 @@ static __global__ void mac_beta_from_rho_kernel(MGeomK g, int d, const double* _
         dt / (0.5 * (rho[cidx(g, L[0], L[1], L[2])] + rho[cidx(g, R[0], R[1], R[2])]));
 }
 
-// ---- bottom: BiCGStab in one workgroup on the MAC operator (FP64) ----
+// The rows of the MAC operator for the bottom solve; its smoothing sweeps are
+// red-black like the V-cycle's, each colour updated from the values before it
+// (cells of one colour meet across a periodic wrap of odd length).
 template <class T>
-__device__ void mac_bottom_apply(const MGeomK& g, const MCoef<double>& c, const T* bx, const T* by,
-                                 const T* bz, const T* a, const double* x, double* y, long n) {
-    __syncthreads();
-    for (long id = threadIdx.x; id < n; id += blockDim.x) {
-        const int q = (int)(id / g.n[0]);
-        const int i = (int)(id - (long)q * g.n[0]);
-        const int j = q % g.n[1];
-        const int k = q / g.n[1];
-        double dg;
-        y[id] = mac_apply_cell<double, T, double>(g, c, bx, by, bz, a, x, i, j, k, dg);
-    }
-    __syncthreads();
-}
-
-// The MAC operator in FP64 for the bottom solve; its smoother is the
-// red-black sweep of the V-cycle, each colour updated from the values before
-// it (cells of one colour meet across a periodic wrap of odd length).
-template <class T>
-struct MacBottomOp {
+struct MacRows {
+    static constexpr int NS = 7;
+    static constexpr bool kRedBlack = true;
     MGeomK g;
     MCoef<double> c;
     const T *bx, *by, *bz, *a;
-    __device__ long size() const { return (long)g.n[0] * g.n[1] * g.n[2]; }
-    __device__ bool held(long) const { return false; }
-    __device__ double nfree() const { return (double)size(); }
-    __device__ void apply(const double* x, double* y, long n) const {
-        mac_bottom_apply<T>(g, c, bx, by, bz, a, x, y, n);
-    }
-    __device__ void smooth(const BottomVecs& V, long n) const {
-        for (int color = 0; color < 2; ++color) {
-            __syncthreads();
-            for (long id = threadIdx.x; id < n; id += blockDim.x) {
-                const int q = (int)(id / g.n[0]);
-                const int i = (int)(id - (long)q * g.n[0]);
-                const int j = q % g.n[1];
-                const int k = q / g.n[1];
-                double u = V.x[id];
-                if (((i + j + k) & 1) == color) {
-                    double dg;
-                    const double acc = mac_apply_cell<double, T, double>(g, c, bx, by, bz, a, V.x,
-                                                                         i, j, k, dg);
-                    if (dg != 0.0) u += (V.b[id] - acc) / dg;
-                }
-                V.t[id] = u;
-            }
-            __syncthreads();
-            for (long id = threadIdx.x; id < n; id += blockDim.x) V.x[id] = V.t[id];
+    __device__ int dim(int d) const { return g.n[d]; }
+    __device__ int per(int d) const { return g.per[d]; }
+    __device__ bool row(int id, int i, int j, int k, double (&C)[NS]) const {
+        const int p[3] = {i, j, k};
+        const T* beta[3] = {bx, by, bz};
+        double dg = a ? -(double)a[id] : 0.0;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            int q[3] = {i, j, k};
+            const double bl = c.ih2[d] * (double)beta[d][fidx(g, d, q[0], q[1], q[2])];
+            q[d] += 1;
+            const double bh = c.ih2[d] * (double)beta[d][fidx(g, d, q[0], q[1], q[2])];
+            const bool il = p[d] > 0 || g.per[d], ih = p[d] + 1 < g.n[d] || g.per[d];
+            C[1 + 2 * d] = il ? bl : 0.0;
+            C[2 + 2 * d] = ih ? bh : 0.0;
+            dg -= il ? bl : (g.dlo[d] ? 2 * bl : 0.0);
+            dg -= ih ? bh : (g.dhi[d] ? 2 * bh : 0.0);
         }
-        __syncthreads();
+        C[0] = dg;
+        return true;
     }
 };
 
-template <class T>
-static __global__ void __launch_bounds__(1024) mac_bottom_kernel(MGeomK g, MCoef<double> c,
-                                                                 const T* bx, const T* by,
-                                                                 const T* bz, const T* a,
-                                                                 const T* b_in,
-                                                                 T* x_out, double* work, int kind,
-                                                                 int maxiter, double rtol,
-                                                                 int singular, int* iters_acc) {
-    __shared__ double red[16];
-    const MacBottomOp<T> op{g, c, bx, by, bz, a};
-    bottom_solve_body(op, b_in, x_out, work, kind, maxiter, rtol, singular, iters_acc, red);
-}
+MGX_BOTTOM_INSTANCE(extern, MacRows<float>, float);
+MGX_BOTTOM_INSTANCE(extern, MacRows<double>, double);
 
 // ---- Robin domain faces: a phi + b dphi/dn = f ---------------------------
 // The face value of phi is the mean of the boundary cell and its ghost and

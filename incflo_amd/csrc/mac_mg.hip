@@ -53,7 +53,8 @@ void MacHierarchy<T>::build(const MacGeom& g0, int nlev) {
         lv.x = lv.x_buf.template as<T>();
         lv.r = lv.r_buf.template as<T>();
     }
-    bottom_work.alloc(7 * L.back().g.ncell() * sizeof(double));
+    bottom_work.alloc(bottom_work_doubles(L.back().g.ncell(), 7) * sizeof(double));
+    bottom_prepare<MacRows<T>, T>();
     built = true;
 }
 
@@ -216,14 +217,15 @@ void MacHierarchy<T>::vcycle_body(const MGOpts& o, hipStream_t s, int* bottom_it
     if (lc < nl - 1) mac_coarse_cycle_kernel<T><<<1, 1024, 0, s>>>(mac_coarse_args(L, lc, o, 0));
     {
         MacLevel<T>& lb = L[nl - 1];
-        const long nb = lb.g.ncell();
-        const int threads = nb >= 1024 ? 1024 : (nb >= 256 ? 256 : 64);
-        mac_bottom_kernel<T><<<1, threads, 0, s>>>(lb.kg, make_mcoef<double>(lb.g.dx), lb.beta[0],
-                                                   lb.beta[1], lb.beta[2], lb.a, lb.b, lb.x,
-                                                   bottom_work.as<double>(), o.bottom_solver,
-                                                   o.bottom_maxiter,
-                                                   o.bottom_rtol, lb.g.singular() ? 1 : 0,
-                                                   bottom_iters);
+        BottomArgs ba{};
+        ba.work = bottom_work.as<double>();
+        ba.kind = o.bottom_solver;
+        ba.maxiter = o.bottom_maxiter;
+        ba.rtol = o.bottom_rtol;
+        ba.singular = lb.g.singular() ? 1 : 0;
+        ba.iters_acc = bottom_iters;
+        const MacRows<T> rows{lb.kg, make_mcoef<double>(lb.g.dx), lb.beta[0], lb.beta[1], lb.beta[2], lb.a};
+        bottom_launch<MacRows<T>, T>(rows, lb.g.ncell(), lb.b, lb.x, ba, s);
     }
     x0_guess = false;
     if (lc < nl - 1) mac_coarse_cycle_kernel<T><<<1, 1024, 0, s>>>(mac_coarse_args(L, lc, o, 1));

@@ -1473,32 +1473,6 @@ static __global__ void zero_dirichlet_kernel(KGeom g, T* __restrict__ a) {
     if (is_dir(g, i, j, k)) a[i + (long)g.nn[0] * (j + (long)g.nn[1] * k)] = 0;
 }
 
-// ---- bottom solve: BiCGStab (van der Vorst 1992) in one workgroup, FP64 ----
-__device__ __forceinline__ double bsum(double v, double* red) {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    const int tid = threadIdx.x;
-    __syncthreads();
-    if ((tid & 63) == 0) red[tid >> 6] = v;
-    __syncthreads();
-    double s = 0.0;
-    const int nw = blockDim.x >> 6;
-    for (int w = 0; w < nw; ++w) s += red[w];
-    return s;
-}
-
-__device__ __forceinline__ double bmax(double v, double* red) {
-    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
-    const int tid = threadIdx.x;
-    __syncthreads();
-    if ((tid & 63) == 0) red[tid >> 6] = v;
-    __syncthreads();
-    double s = 0.0;
-    const int nw = blockDim.x >> 6;
-    for (int w = 0; w < nw; ++w) s = fmax(s, red[w]);
-    return s;
-}
-
-// (L x)_n with direct loads, in double; Dirichlet rows masked to 0.
 // (L x)_n with direct loads of the 3x3x3 neighbourhood, in TO precision
 // (same unrolled arithmetic as the streaming kernel).
 template <class TO, class TS, class TX>
@@ -1531,492 +1505,10 @@ __device__ __forceinline__ TO apply_node_nbhd(const KGeom& g, const Coef<TO>& c,
                : apply27<TO, false, 0>(P[0], P[1], P[2], S[0], S[1], c, ssum);
 }
 
-// (L x)_n in double; Dirichlet rows masked to 0.
-template <class TS>
-__device__ double apply_node_direct(const KGeom& g, const Coef<double>& c, const TS* sig,
-                                    const double* x, int i, int j, int k) {
-    if (is_dir(g, i, j, k)) return 0.0;
-    double ssum;
-    return apply_node_nbhd<double, TS, double>(g, c, sig, x, i, j, k, ssum);
-}
-
 // A node held at zero: a Dirichlet node, or mask 0 of an overset mask (m may be null).
 __device__ __forceinline__ bool node_fixed(const KGeom& g, const unsigned char* m, long id, int i,
                                            int j, int k) {
     return is_dir(g, i, j, k) || (m && !m[id]);
-}
-
-template <class TS>
-__device__ void bottom_apply(const KGeom& g, const Coef<double>& c, const TS* sig,
-                             const unsigned char* m, const double* x, double* y, long n) {
-    __syncthreads();
-    for (long id = threadIdx.x; id < n; id += blockDim.x) {
-        const int i = id % g.nn[0];
-        const int j = (id / g.nn[0]) % g.nn[1];
-        const int k = id / ((long)g.nn[0] * g.nn[1]);
-        y[id] = (m && !m[id]) ? 0.0 : apply_node_direct(g, c, sig, x, i, j, k);
-    }
-    __syncthreads();
-}
-
-// The bottom_solver choices of MLMG (MGX_BOTTOM_*): BiCGStab (van der Vorst
-// 1992), CG (Hestenes and Stiefel 1952), BiCGStab and then CG from zero when
-// the first one fails ("bicgcg"), the reverse ("cgbicg"), or smoothing sweeps
-// only ("smoother").  A Krylov solve that does not reach rtol is followed by
-// kBottomSmooths smoothing sweeps, from zero when it broke down (a zero
-// inner product).  Both operators are negative (semi-)definite and
-// symmetric, so CG applies as it stands.
-constexpr int kBottomSmooths = 8;
-
-// the 7 FP64 work vectors of the bottom solve
-struct BottomVecs {
-    double *x, *r, *b, *p, *v, *s, *t;
-};
-
-__device__ __forceinline__ BottomVecs bottom_vecs(double* w, long n) {
-    return BottomVecs{w, w + n, w + 2 * n, w + 3 * n, w + 4 * n, w + 5 * n, w + 6 * n};
-}
-
-// 0: converged, 1: broke down, 2: iteration limit.  Starts from x = 0.
-template <class Op>
-__device__ int bottom_bicgstab(const Op& op, const BottomVecs& V, long n, int maxiter,
-                               double rtol, double rnorm0, int& iters, double* red) {
-    const int tid = threadIdx.x, nt = blockDim.x;
-    double *x = V.x, *r = V.r, *rh = V.b, *p = V.p, *v = V.v, *s = V.s, *t = V.t;
-    for (long id = tid; id < n; id += nt) {
-        r[id] = rh[id];
-        x[id] = 0.0; p[id] = 0.0; v[id] = 0.0;
-    }
-    double rho = 1.0, alpha = 1.0, omega = 1.0;
-    for (int it = 1; it <= maxiter; ++it) {
-        iters = it;
-        double q = 0.0;
-        for (long id = tid; id < n; id += nt) q += rh[id] * r[id];
-        const double rho_new = bsum(q, red);
-        if (rho_new == 0.0) return 1;
-        const double beta = (rho_new / rho) * (alpha / omega);
-        for (long id = tid; id < n; id += nt) p[id] = r[id] + beta * (p[id] - omega * v[id]);
-        op.apply(p, v, n);
-        q = 0.0;
-        for (long id = tid; id < n; id += nt) q += rh[id] * v[id];
-        const double rhv = bsum(q, red);
-        if (rhv == 0.0) return 1;
-        alpha = rho_new / rhv;
-        double sn = 0.0;
-        for (long id = tid; id < n; id += nt) {
-            x[id] += alpha * p[id];
-            s[id] = r[id] - alpha * v[id];
-            sn = fmax(sn, nabs(s[id]));
-        }
-        sn = bmax(sn, red);
-        if (sn <= rtol * rnorm0) return 0;
-        op.apply(s, t, n);
-        double tt = 0.0, ts = 0.0;
-        for (long id = tid; id < n; id += nt) { tt += t[id] * t[id]; ts += t[id] * s[id]; }
-        tt = bsum(tt, red);
-        ts = bsum(ts, red);
-        if (tt == 0.0) return 1;
-        omega = ts / tt;
-        double rr = 0.0;
-        for (long id = tid; id < n; id += nt) {
-            x[id] += omega * s[id];
-            r[id] = s[id] - omega * t[id];
-            rr = fmax(rr, nabs(r[id]));
-        }
-        rr = bmax(rr, red);
-        if (rr <= rtol * rnorm0) return 0;
-        if (omega == 0.0) return 1;
-        rho = rho_new;
-    }
-    return 2;
-}
-
-// Conjugate gradients from x = 0; same return codes.
-template <class Op>
-__device__ int bottom_cg(const Op& op, const BottomVecs& V, long n, int maxiter, double rtol,
-                         double rnorm0, int& iters, double* red) {
-    const int tid = threadIdx.x, nt = blockDim.x;
-    double *x = V.x, *r = V.r, *p = V.p, *v = V.v;
-    for (long id = tid; id < n; id += nt) {
-        r[id] = V.b[id];
-        x[id] = 0.0; p[id] = 0.0;
-    }
-    double rho_old = 1.0;
-    for (int it = 1; it <= maxiter; ++it) {
-        iters = it;
-        double q = 0.0;
-        for (long id = tid; id < n; id += nt) q += r[id] * r[id];
-        const double rho = bsum(q, red);
-        if (rho == 0.0) return 0;  // the residual vanished
-        const double beta = it == 1 ? 0.0 : rho / rho_old;
-        for (long id = tid; id < n; id += nt) p[id] = r[id] + beta * p[id];
-        op.apply(p, v, n);
-        q = 0.0;
-        for (long id = tid; id < n; id += nt) q += p[id] * v[id];
-        const double pv = bsum(q, red);
-        if (pv == 0.0) return 1;
-        const double alpha = rho / pv;
-        double rn = 0.0;
-        for (long id = tid; id < n; id += nt) {
-            x[id] += alpha * p[id];
-            r[id] -= alpha * v[id];
-            rn = fmax(rn, nabs(r[id]));
-        }
-        rn = bmax(rn, red);
-        if (rn <= rtol * rnorm0) return 0;
-        rho_old = rho;
-    }
-    return 2;
-}
-
-// The bottom solve of op's level: b_in (mean-free over the free unknowns when
-// singular, zero at held ones) -> x_out (likewise; zero at held unknowns).
-// Adds the Krylov iterations (or smoothing sweeps) to *iters_acc.
-template <class Op, class T>
-__device__ void bottom_solve_body(const Op& op, const T* b_in, T* x_out, double* work, int kind,
-                                  int maxiter, double rtol, int singular, int* iters_acc,
-                                  double* red) {
-    const long n = op.size();
-    const BottomVecs V = bottom_vecs(work, n);
-    const int tid = threadIdx.x, nt = blockDim.x;
-    double bs = 0.0;
-    for (long id = tid; id < n; id += nt) {
-        V.b[id] = op.held(id) ? 0.0 : (double)b_in[id];
-        bs += V.b[id];
-    }
-    bs = bsum(bs, red);
-    const double nfree = op.nfree();
-    const double bmean = (singular && nfree > 0.0) ? bs / nfree : 0.0;
-    double rn = 0.0;
-    for (long id = tid; id < n; id += nt) {
-        if (!op.held(id)) V.b[id] -= bmean;
-        V.x[id] = 0.0;
-        rn = fmax(rn, nabs(V.b[id]));
-    }
-    const double rnorm0 = bmax(rn, red);
-    int it = 0;
-    if (rnorm0 > 0.0) {
-        int st = 2, smooths = 0;
-        if (kind == MGX_BOTTOM_SMOOTHER) {
-            smooths = kBottomSmooths;
-        } else {
-            const bool cg_first = kind == MGX_BOTTOM_CG || kind == MGX_BOTTOM_CGBICG;
-            st = cg_first ? bottom_cg(op, V, n, maxiter, rtol, rnorm0, it, red)
-                          : bottom_bicgstab(op, V, n, maxiter, rtol, rnorm0, it, red);
-            if (st != 0 && (kind == MGX_BOTTOM_BICGCG || kind == MGX_BOTTOM_CGBICG)) {
-                int it2 = 0;
-                st = cg_first ? bottom_bicgstab(op, V, n, maxiter, rtol, rnorm0, it2, red)
-                              : bottom_cg(op, V, n, maxiter, rtol, rnorm0, it2, red);
-                it += it2;
-            }
-            if (st != 0) smooths = kBottomSmooths;
-        }
-        if (st == 1)
-            for (long id = tid; id < n; id += nt) V.x[id] = 0.0;
-        for (int q = 0; q < smooths; ++q) op.smooth(V, n);
-        if (kind == MGX_BOTTOM_SMOOTHER) it = smooths;
-    }
-    __syncthreads();
-    double xs = 0.0;
-    for (long id = tid; id < n; id += nt) xs += op.held(id) ? 0.0 : V.x[id];
-    xs = bsum(xs, red);
-    const double xmean = (singular && nfree > 0.0) ? xs / nfree : 0.0;
-    for (long id = tid; id < n; id += nt) x_out[id] = op.held(id) ? (T)0 : (T)(V.x[id] - xmean);
-    if (tid == 0 && iters_acc) atomicAdd(iters_acc, it);
-}
-
-// The nodal operator in FP64 for the bottom solve; its smoother is the
-// weighted Jacobi sweep of the V-cycle.
-template <class TS>
-struct NodalBottomOp {
-    KGeom g;
-    Coef<double> c;
-    const TS* sig;
-    const unsigned char* m;  // overset mask, may be null
-    double omega;
-    __device__ long size() const { return (long)g.nn[0] * g.nn[1] * g.nn[2]; }
-    __device__ bool held(long id) const { return m && !m[id]; }
-    // a singular problem has no held nodes (a mask that holds one makes it regular)
-    __device__ double nfree() const { return (double)size(); }
-    __device__ void apply(const double* x, double* y, long n) const {
-        bottom_apply(g, c, sig, m, x, y, n);
-    }
-    __device__ void smooth(const BottomVecs& V, long n) const {
-        __syncthreads();
-        for (long id = threadIdx.x; id < n; id += blockDim.x) {
-            const int i = id % g.nn[0];
-            const int j = (id / g.nn[0]) % g.nn[1];
-            const int k = id / ((long)g.nn[0] * g.nn[1]);
-            double ssum;
-            const double acc = apply_node_nbhd<double, TS, double>(g, c, sig, V.x, i, j, k, ssum);
-            double u = V.x[id];
-            if (node_fixed(g, m, id, i, j, k)) u = 0.0;
-            else if (ssum != 0.0) u += omega * (V.b[id] - acc) / (-c.diag4 * ssum);
-            V.t[id] = u;
-        }
-        __syncthreads();
-        for (long id = threadIdx.x; id < n; id += blockDim.x) V.x[id] = V.t[id];
-        __syncthreads();
-    }
-};
-
-template <class T>
-static __global__ void __launch_bounds__(1024) bottom_solve_kernel(KGeom g, Coef<double> c,
-                                                                   const T* sig,
-                                                                   const unsigned char* m,
-                                                                   const T* b_in, T* x_out,
-                                                                   double* work, int kind,
-                                                                   int maxiter, double rtol,
-                                                                   double omega, int singular,
-                                                                   int* iters_acc) {
-    __shared__ double red[16];
-    const NodalBottomOp<T> op{g, c, sig, m, omega};
-    bottom_solve_body(op, b_in, x_out, work, kind, maxiter, rtol, singular, iters_acc, red);
-}
-
-// ---- coarse levels: the whole V-cycle below a size threshold in one workgroup ----
-// The levels are small enough that one workgroup sweeps each of them in a few
-// microseconds, so running smoothing, residual, restriction, prolongation and
-// the BiCGStab bottom solve back to back with workgroup barriers replaces
-// about 7 launches per level.  Same operations, same order, as the per-level
-// kernels.
-constexpr int kMaxCoarse = 8;
-
-template <class T>
-struct CoarseLevel {
-    KGeom g;
-    Coef<T> c;
-    T omega;
-    const T* sig;
-    T* b;
-    T* x;
-    T* x2;
-    T* r;
-    const unsigned char* m;  // overset mask (global memory), null without one
-};
-
-template <class T>
-struct CoarseArgs {
-    CoarseLevel<T> L[kMaxCoarse];
-    int nl;           // levels in this launch (the last one is the bottom)
-    int nu1, nu2;
-    Coef<double> cb;  // bottom operator coefficients (double)
-    double* work;
-    int bottom_kind;  // MGX_BOTTOM_*
-    double bottom_omega;
-    int maxiter;
-    double rtol;
-    int singular;
-    int* iters_acc;
-};
-
-template <class T>
-__device__ __forceinline__ void node_of(const KGeom& g, int id, int& i, int& j, int& k) {
-    const int q = id / g.nn[0];
-    i = id - q * g.nn[0];
-    j = q % g.nn[1];
-    k = q / g.nn[1];
-}
-
-// L x at node (i,j,k) with direct loads; also returns the sum of the 8 cell coefficients.
-template <class T>
-__device__ __forceinline__ T apply_node_T(const KGeom& g, const Coef<T>& c, const T* sig,
-                                          const T* x, int i, int j, int k, T& ssum) {
-    return apply_node_nbhd<T, T, T>(g, c, sig, x, i, j, k, ssum);
-}
-
-// Bytes of dynamic LDS the coarse kernel needs for levels L[0..nl-1]: every
-// level's sigma, b, x, x2 and r (r shares x2's storage) and the bottom
-// solver's 7 FP64 work vectors.
-template <class T>
-inline size_t coarse_lds_bytes(const KGeom* g, int nl) {
-    size_t b = 0;
-    for (int l = 0; l < nl; ++l) {
-        const size_t nn = (size_t)g[l].nn[0] * g[l].nn[1] * g[l].nn[2];
-        const size_t ns = (size_t)g[l].sg[0] * g[l].sg[1] * g[l].sg[2];
-        b += ((ns + 3 * nn) * sizeof(T) + 15) / 16 * 16;
-    }
-    const size_t nb = (size_t)g[nl - 1].nn[0] * g[nl - 1].nn[1] * g[nl - 1].nn[2];
-    return b + 7 * nb * sizeof(double);
-}
-
-// The whole coarse hierarchy lives in LDS for the duration of the launch:
-// sigma and the top level's rhs are copied in, the top level's correction is
-// copied out; everything in between never touches global memory.
-template <class T>
-static __global__ void __launch_bounds__(512) coarse_vcycle_kernel(const CoarseArgs<T> a) {
-    __shared__ double red[16];
-    __shared__ CoarseLevel<T> sl[kMaxCoarse];  // level descriptors with LDS pointers
-    __shared__ double* swork;
-    extern __shared__ __align__(16) unsigned char lds[];
-    const int tid = threadIdx.x, nt = blockDim.x;
-    if (tid == 0) {
-        size_t off = 0;
-        for (int l = 0; l < a.nl; ++l) {
-            CoarseLevel<T> lv = a.L[l];
-            const int nn = lv.g.nn[0] * lv.g.nn[1] * lv.g.nn[2];
-            const int ns = lv.g.sg[0] * lv.g.sg[1] * lv.g.sg[2];
-            T* base = reinterpret_cast<T*>(lds + off);
-            lv.sig = base;
-            lv.b = base + ns;
-            lv.x = base + ns + nn;
-            lv.x2 = base + ns + 2 * nn;
-            lv.r = lv.x2;  // the residual is formed after smoothing, when x2 is free
-            sl[l] = lv;
-            off += ((size_t)(ns + 3 * nn) * sizeof(T) + 15) / 16 * 16;
-        }
-        swork = reinterpret_cast<double*>(lds + off);
-    }
-    __syncthreads();
-    for (int l = 0; l < a.nl; ++l) {
-        const int ns = sl[l].g.sg[0] * sl[l].g.sg[1] * sl[l].g.sg[2];
-        T* dst = const_cast<T*>(sl[l].sig);
-        const T* src = a.L[l].sig;
-        for (int id = tid; id < ns; id += nt) dst[id] = src[id];
-    }
-    {
-        const int nn = sl[0].g.nn[0] * sl[0].g.nn[1] * sl[0].g.nn[2];
-        for (int id = tid; id < nn; id += nt) sl[0].b[id] = a.L[0].b[id];
-    }
-    __syncthreads();
-    T* top_x_global = a.L[0].x;
-    unsigned swmask = 0u;  // bit l: level l's current iterate is in x2
-    auto cur = [&](int l) { return ((swmask >> l) & 1u) ? sl[l].x2 : sl[l].x; };
-    auto oth = [&](int l) { return ((swmask >> l) & 1u) ? sl[l].x : sl[l].x2; };
-    auto jacobi = [&](int l) {
-        const CoarseLevel<T>& lv = sl[l];
-        const int n = lv.g.nn[0] * lv.g.nn[1] * lv.g.nn[2];
-        const T* xin = cur(l);
-        T* xout = oth(l);
-        for (int id = tid; id < n; id += nt) {
-            int i, j, k;
-            node_of<T>(lv.g, id, i, j, k);
-            T ssum;
-            const T acc = apply_node_T<T>(lv.g, lv.c, lv.sig, xin, i, j, k, ssum);
-            T v = xin[id];
-            if (node_fixed(lv.g, lv.m, id, i, j, k)) v = 0;
-            else if (ssum != (T)0) v = v + lv.omega * (lv.b[id] - acc) / (-lv.c.diag4 * ssum);
-            xout[id] = v;
-        }
-        swmask ^= (1u << l);
-        __syncthreads();
-    };
-    // down
-    for (int l = 0; l < a.nl - 1; ++l) {
-        const CoarseLevel<T>& lv = sl[l];
-        const int n = lv.g.nn[0] * lv.g.nn[1] * lv.g.nn[2];
-        if (a.nu1 > 0) {
-            T* x = cur(l);
-            for (int id = tid; id < n; id += nt) {
-                int i, j, k;
-                node_of<T>(lv.g, id, i, j, k);
-                T ssum = 0;
-                for (int q = 0; q < 8; ++q)
-                    ssum += lv.sig[(i + (q & 1)) + (long)lv.g.sg[0] * ((j + ((q >> 1) & 1)) +
-                                                                    (long)lv.g.sg[1] * (k + ((q >> 2) & 1)))];
-                x[id] = (node_fixed(lv.g, lv.m, id, i, j, k) || ssum == (T)0)
-                            ? (T)0
-                            : lv.omega * lv.b[id] / (-lv.c.diag4 * ssum);
-            }
-            __syncthreads();
-            for (int s = 1; s < a.nu1; ++s) jacobi(l);
-        } else {
-            T* x = cur(l);
-            for (int id = tid; id < n; id += nt) x[id] = 0;
-            __syncthreads();
-        }
-        {
-            const T* x = cur(l);
-            for (int id = tid; id < n; id += nt) {
-                int i, j, k;
-                node_of<T>(lv.g, id, i, j, k);
-                T ssum;
-                const T acc = apply_node_T<T>(lv.g, lv.c, lv.sig, x, i, j, k, ssum);
-                oth(l)[id] = node_fixed(lv.g, lv.m, id, i, j, k) ? (T)0 : lv.b[id] - acc;
-            }
-            __syncthreads();
-        }
-        {
-            const CoarseLevel<T>& cv = sl[l + 1];
-            const T* rf = oth(l);  // the residual just formed
-            const KGeom& gf = lv.g;
-            const KGeom& gc = cv.g;
-            const int nc = gc.nn[0] * gc.nn[1] * gc.nn[2];
-            for (int id = tid; id < nc; id += nt) {
-                int I, J, K;
-                node_of<T>(gc, id, I, J, K);
-                T acc = 0;
-                if (!node_fixed(gc, cv.m, id, I, J, K)) {
-                    for (int oz = -1; oz <= 1; ++oz) {
-                        int fk = 2 * K + oz;
-                        if (gf.per[2]) fk = fk < 0 ? fk + gf.nn[2] : (fk >= gf.nn[2] ? fk - gf.nn[2] : fk);
-                        else if (fk < 0 || fk >= gf.nn[2]) continue;
-                        for (int oy = -1; oy <= 1; ++oy) {
-                            int fj = 2 * J + oy;
-                            if (gf.per[1]) fj = fj < 0 ? fj + gf.nn[1] : (fj >= gf.nn[1] ? fj - gf.nn[1] : fj);
-                            else if (fj < 0 || fj >= gf.nn[1]) continue;
-                            for (int ox = -1; ox <= 1; ++ox) {
-                                int fi = 2 * I + ox;
-                                if (gf.per[0]) fi = fi < 0 ? fi + gf.nn[0] : (fi >= gf.nn[0] ? fi - gf.nn[0] : fi);
-                                else if (fi < 0 || fi >= gf.nn[0]) continue;
-                                const T w = (ox ? (T)0.25 : (T)0.5) * (oy ? (T)0.25 : (T)0.5) *
-                                            (oz ? (T)0.25 : (T)0.5);
-                                acc += w * rf[fi + (long)gf.nn[0] * (fj + (long)gf.nn[1] * fk)];
-                            }
-                        }
-                    }
-                }
-                cv.b[id] = acc;
-            }
-            __syncthreads();
-        }
-    }
-    // bottom
-    {
-        const int lb = a.nl - 1;
-        const NodalBottomOp<T> op{sl[lb].g, a.cb, sl[lb].sig, sl[lb].m, a.bottom_omega};
-        bottom_solve_body(op, sl[lb].b, cur(lb), swork, a.bottom_kind, a.maxiter, a.rtol,
-                          a.singular, a.iters_acc, red);
-        __syncthreads();
-    }
-    // up
-    for (int l = a.nl - 2; l >= 0; --l) {
-        const CoarseLevel<T>& lv = sl[l];
-        const KGeom& gf = lv.g;
-        const KGeom& gc = sl[l + 1].g;
-        const T* xc = cur(l + 1);
-        T* xf = cur(l);
-        const int nf = gf.nn[0] * gf.nn[1] * gf.nn[2];
-        for (int id = tid; id < nf; id += nt) {
-            int i, j, k;
-            node_of<T>(gf, id, i, j, k);
-            if (node_fixed(gf, lv.m, id, i, j, k)) continue;
-            const int f[3] = {i, j, k};
-            int lo[3], hi[3];
-            for (int d = 0; d < 3; ++d) {
-                lo[d] = f[d] >> 1;
-                hi[d] = (f[d] & 1) ? lo[d] + 1 : lo[d];
-                if (gc.per[d] && hi[d] >= gc.nn[d]) hi[d] -= gc.nn[d];
-            }
-            T acc = 0;
-            for (int q = 0; q < 8; ++q) {
-                const int I = (q & 1) ? hi[0] : lo[0];
-                const int J = (q & 2) ? hi[1] : lo[1];
-                const int K = (q & 4) ? hi[2] : lo[2];
-                acc += xc[I + (long)gc.nn[0] * (J + (long)gc.nn[1] * K)];
-            }
-            xf[id] += (T)0.125 * acc;
-        }
-        __syncthreads();
-        for (int s = 0; s < a.nu2; ++s) jacobi(l);
-    }
-    // the top level's correction goes back to global memory
-    {
-        const CoarseLevel<T>& lv = sl[0];
-        const int n = lv.g.nn[0] * lv.g.nn[1] * lv.g.nn[2];
-        const T* xs = cur(0);
-        for (int id = tid; id < n; id += nt) top_x_global[id] = xs[id];
-    }
 }
 
 }  // namespace mgx

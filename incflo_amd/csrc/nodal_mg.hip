@@ -23,6 +23,7 @@
 #include "eb_nodal.h"
 #include "learned_kernels.h"
 #include "mgx_ctx.h"
+#include "nodal_coarse.h"
 #include "nodal_mg.h"
 
 namespace mgx {
@@ -408,6 +409,7 @@ void NodalHierarchy<T>::build(const NodalGeom& g0, int nlev) {
         // any stream capture
         (void)hipFuncSetAttribute((const void*)coarse_vcycle_kernel<T>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024);
+        bottom_prepare<NodalRows<T>, T>();
         attr_set = true;
     }
     L.clear();
@@ -431,7 +433,7 @@ void NodalHierarchy<T>::build(const NodalGeom& g0, int nlev) {
         lv.x2 = lv.x2_buf.template as<T>();
         lv.r = lv.r_buf.template as<T>();
     }
-    bottom_work.alloc(7 * L.back().g.nnode() * sizeof(double));
+    bottom_work.alloc(bottom_work_doubles(L.back().g.nnode(), 27) * sizeof(double));
     built = true;
 }
 
@@ -608,7 +610,8 @@ void NodalHierarchy<T>::vcycle(const MGOpts& o, hipStream_t s, int* bottom_iters
 template <class T>
 void NodalHierarchy<T>::vcycle_body(const MGOpts& o, hipStream_t s, int* bottom_iters) {
     const int nl = (int)L.size();
-    // levels lc..nl-1 run in the LDS-resident coarse kernel (when they fit)
+    // levels lc..nl-1 run in the LDS-resident coarse kernel (tuning table
+    // coarse_nodes, when they fit); lc == nl - 1: the bottom solve alone
     constexpr size_t kLdsBudget = 150 * 1024;
     auto lds_for = [&](int first) {
         KGeom gs[kMaxCoarse];
@@ -616,11 +619,9 @@ void NodalHierarchy<T>::vcycle_body(const MGOpts& o, hipStream_t s, int* bottom_
         return coarse_lds_bytes<T>(gs, nl - first);
     };
     int lc = nl - 1;
-    const bool bottom_in_lds = lds_for(nl - 1) <= kLdsBudget;
-    if (bottom_in_lds)
-        while (lc > 0 && nl - (lc - 1) <= kMaxCoarse && L[lc - 1].g.nnode() <= coarse_threshold() &&
-               lds_for(lc - 1) <= kLdsBudget)
-            --lc;
+    while (lc > 0 && nl - (lc - 1) <= kMaxCoarse && L[lc - 1].g.nnode() <= coarse_threshold() &&
+           lds_for(lc - 1) <= kLdsBudget)
+        --lc;
     bool ready = x0_ready && o.nu1 > 0;
     const bool guess = x0_guess;
     x0_ready = false;
@@ -646,14 +647,18 @@ void NodalHierarchy<T>::vcycle_body(const MGOpts& o, hipStream_t s, int* bottom_
         launch_restrict<T>(lv.kg, lc1.g, lc1.kg, lv.r, lc1.b, lc1.sig, lc1.coef.diag4,
                            (T)sweep_omega(lc1.g, o, cheb, 0, o.nu1), ready ? lc1.x : nullptr, s);
     }
-    if (!bottom_in_lds) {
-        MGLevel<T>& lb = L[nl - 1];
-        const long nb = lb.g.nnode();
-        const int threads = nb >= 1024 ? 1024 : (nb >= 256 ? 256 : 64);
-        bottom_solve_kernel<T><<<1, threads, 0, s>>>(
-            lb.kg, make_coef<double>(lb.g.dx), lb.sig, mask(nl - 1), lb.b, lb.x,
-            bottom_work.as<double>(), o.bottom_solver, o.bottom_maxiter, o.bottom_rtol,
-            nodal_omega(lb.g, o.omega), bottom_singular() ? 1 : 0, bottom_iters);
+    const MGLevel<T>& lb = L[nl - 1];
+    BottomArgs ba{};
+    ba.work = bottom_work.as<double>();
+    ba.kind = o.bottom_solver;
+    ba.maxiter = o.bottom_maxiter;
+    ba.rtol = o.bottom_rtol;
+    ba.omega = nodal_omega(lb.g, o.omega);
+    ba.singular = bottom_singular() ? 1 : 0;
+    ba.iters_acc = bottom_iters;
+    if (lc == nl - 1) {
+        const NodalRows<T> rows{lb.kg, make_coef<double>(lb.g.dx), lb.sig, mask(nl - 1)};
+        bottom_launch<NodalRows<T>, T>(rows, lb.g.nnode(), lb.b, lb.x, ba, s);
     } else {
         CoarseArgs<T> ca{};
         ca.nl = nl - lc;
@@ -671,17 +676,10 @@ void NodalHierarchy<T>::vcycle_body(const MGOpts& o, hipStream_t s, int* bottom_
             ca.L[q].m = mask(lc + q);
             nmax = std::max(nmax, lv.g.nnode());
         }
-        const MGLevel<T>& lb = L[nl - 1];
         ca.nu1 = o.nu1;
         ca.nu2 = o.nu2;
         ca.cb = make_coef<double>(lb.g.dx);
-        ca.work = bottom_work.as<double>();
-        ca.bottom_kind = o.bottom_solver;
-        ca.bottom_omega = nodal_omega(lb.g, o.omega);
-        ca.maxiter = o.bottom_maxiter;
-        ca.rtol = o.bottom_rtol;
-        ca.singular = bottom_singular() ? 1 : 0;
-        ca.iters_acc = bottom_iters;
+        ca.bottom = ba;
         const int threads = nmax >= 512 ? 512 : (nmax >= 256 ? 256 : 64);
         coarse_vcycle_kernel<T><<<1, threads, lds_for(lc), s>>>(ca);
     }
