@@ -649,6 +649,8 @@ MGX_API int mgx_mac_set_eb_cylinder(mgx_mac h, double cx, double cy, double r) {
         h->eb_cyl[0] = cx;
         h->eb_cyl[1] = cy;
         h->eb_cyl[2] = r;
+        // cut cells on a grid two or three cells wide do not represent the body
+        h->solver.set_deep(false);
         if (!h->dirty) h->build_eb();
     });
 }

@@ -114,6 +114,8 @@ class MacSolver {
     MacGeom g0;
     MGOpts opts;
     int nlev = 1;
+    bool deep = true;     // levels down to 2 cells where the bottom would be large (nodal_nlevels)
+    void set_deep(bool on);
     MacHierarchy<double> H64;
     MacHierarchy<float> H32;
     DevBuf beta0[3];      // level-0 face coefficients (FP64)

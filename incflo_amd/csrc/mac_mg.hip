@@ -246,10 +246,10 @@ MacSolver::~MacSolver() {
     if (h_pinned) (void)hipHostFree(h_pinned);
 }
 
-static int mac_nlevels(const MacGeom& g, int max_coarsening_level) {
+static int mac_nlevels(const MacGeom& g, int max_coarsening_level, bool deep) {
     NodalGeom ng{};
     for (int d = 0; d < 3; ++d) ng.n[d] = g.n[d];
-    return nodal_nlevels(ng, max_coarsening_level);
+    return nodal_nlevels(ng, max_coarsening_level, deep);
 }
 
 void MacSolver::setup(const MacGeom& g, const MGOpts& o) {
@@ -259,7 +259,7 @@ void MacSolver::setup(const MacGeom& g, const MGOpts& o) {
                            g.per[0] == g0.per[0] && g.per[1] == g0.per[1] && g.per[2] == g0.per[2];
     g0 = g;
     opts = o;
-    nlev = mac_nlevels(g, o.max_coarsening_level);
+    nlev = mac_nlevels(g, o.max_coarsening_level, deep);
     for (int d = 0; d < 3; ++d) beta0[d].alloc(g.nface(d) * sizeof(double));
     const long n = g.ncell();
     if (g.has_a) acoef0.alloc(n * sizeof(double));
@@ -278,6 +278,11 @@ void MacSolver::setup(const MacGeom& g, const MGOpts& o) {
     h32_beta = h64_beta = false;
     rob_levels = 0;  // the level count may have changed
     beta0s_ok = false;
+}
+
+void MacSolver::set_deep(bool on) {
+    deep = on;
+    nlev = mac_nlevels(g0, opts.max_coarsening_level, deep);
 }
 
 void MacSolver::set_robin(int d, int side, std::vector<double> a, std::vector<double> b) {

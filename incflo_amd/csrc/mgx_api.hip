@@ -63,7 +63,7 @@ struct mgx_nodal_s {
         if (eb_kind == 0) return;
         if (eb_kind == 1) eb_cylinder_moments(g, prob_lo, eb_cyl[0], eb_cyl[1], eb_cyl[2], eb_type, eb_mom);
         eb = std::make_unique<EBNodal>();
-        eb->setup(g, solver.nlev, eb_type, eb_mom, stream());
+        eb->setup(g, nodal_nlevels(g, opts.max_coarsening_level), eb_type, eb_mom, stream());
         solver.eb = eb.get();
         if (eb_kind == 1) {
             std::vector<double> bw;
