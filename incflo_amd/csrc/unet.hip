@@ -411,7 +411,7 @@ void UNet::backward(const float* in, const float* dout, const NetShape& sh) {
         head_bwd_kernel<<<hb, 256, 0, stream>>>(A(s0 + 2), base, n0, P + head_w, dout, GA(s0 + 2),
                                                 gws.as<float>());
         MGX_REQUIRE(head_b == head_w + base, MGX_ERR_STATE, "U-net: head parameter layout");
-        sum_parts_kernel<<<1, 256, 0, stream>>>(gws.as<float>(), (int)hb, base + 1, G + head_w);
+        sum_parts_kernel<<<(unsigned)(base + 1), 256, 0, stream>>>(gws.as<float>(), (int)hb, base + 1, G + head_w);
     }
     // decoder, finest first
     int li_dec = (int)conv.size() - 2;  // index of dec level 0 conv a

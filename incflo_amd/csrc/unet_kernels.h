@@ -348,117 +348,202 @@ inline void conv3d_forward_launch(const ConvGeom& cg, const float* in, const uns
 
 // Weight gradient: part[chunk][co][k] = sum over the chunk's voxels v of
 // dY[v][co] * A[v][k] (row stride kp); conv3d_dw_reduce_kernel adds the
-// chunks in a fixed order, so training is reproducible.  One wave owns one
-// 16 (co) x 16 (k) tile and one chunk of voxels.
-static __global__ void __launch_bounds__(64) conv3d_dw_kernel(ConvGeom g, const float* __restrict__ in,
-                                                              const float* __restrict__ dy,
-                                                              float* __restrict__ part, int vchunk) {
-    const int lane = threadIdx.x;
+// chunks in a fixed order, so training is reproducible.
+//
+// The products contract over voxels, so both MFMA operands need 8 consecutive
+// voxels of one channel, which channels-last tensors scatter: read per lane
+// from global memory (8 + 8 scalar loads with the index arithmetic of every
+// tap) the kernel took 3.7 ms of a 8 x 32^3 training batch.  Here a workgroup
+// owns 16 NCO output channels x CB input channels x all 27 taps over a range of
+// 4 x 4 x 4 voxel tiles; per tile it transposes dY (BF16 [8 voxels] runs) and
+// the 6 x 6 x 6 halo (BF16 runs of 4 voxels along x, one copy per x offset of
+// the taps, so every run is aligned) into LDS and reads each fragment with
+// 8- or 16-byte loads.  A fragment of the halo serves NCO products.  Bound by
+// the staging (3 halo copies), about 10 times the matrix instructions' time:
+// 3720 -> 350 us for the batch's 14 layers.
+template <int CB, int NCO>
+static __global__ void __launch_bounds__(256) conv3d_dw_kernel(ConvGeom g, const float* __restrict__ in,
+                                                               const float* __restrict__ dy,
+                                                               float* __restrict__ part, int nchunk,
+                                                               int gx, int gy, int gz) {
+    constexpr int NT = (27 * CB + 15) / 16, NTW = (NT + 3) / 4, CO = 16 * NCO;
+    __shared__ __align__(16) unsigned short xs[3][36][CB][4];  // [x offset][halo row][channel][x]
+    __shared__ __align__(16) unsigned short ys[8][CO][8];      // [voxel octet][channel][voxel]
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int row = lane & 15, kq = lane >> 4;
-    const int ntk = g.kp / 16;
-    const int tile = blockIdx.x % (ntk * (g.cout / 16));
-    const int chunk = blockIdx.x / (ntk * (g.cout / 16));
-    const int co0 = (tile / ntk) * 16, kk0 = (tile % ntk) * 16;
+    const int nci = g.cin / CB, nblk = nci * (g.cout / CO);
+    const int chunk = blockIdx.x / nblk, blk = blockIdx.x % nblk;
+    const int ci0 = (blk % nci) * CB, co0 = (blk / nci) * CO;
     const long S = (long)g.nx * g.ny * g.nz;
-    const long nvox = S * g.batch;
-    const long vbeg = (long)chunk * vchunk;
-    const long vend = vbeg + vchunk < nvox ? vbeg + vchunk : nvox;
-    const int K = 27 * g.cin;
-    // this lane's B column: k = kk0 + row
-    const int kcol = kk0 + row;
-    int tap = 0, ci = 0, dz = 0, dyo = 0, dx = 0;
-    const bool kok = kcol < K;
-    if (kok) {
-        tap = kcol / g.cin;
-        ci = kcol - tap * g.cin;
-        dz = tap / 9 - 1;
-        dyo = (tap / 3) % 3 - 1;
-        dx = tap % 3 - 1;
-    }
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (long vb = vbeg; vb < vend; vb += 32) {
-        bf16x8 a, bb;
+    const long ntile = (long)gx * gy * gz * g.batch;
+    const long tbeg = ntile * chunk / nchunk, tend = ntile * (chunk + 1) / nchunk;
+    // B column k = 16 nt + row = tap CB + channel: its run in xs for halo row 0
+    int boff[NTW];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const long v = vb + 8 * kq + i;
-            float av = 0.f, bv = 0.f;
-            if (v < vend) {
-                av = dy[v * g.cout + co0 + row];
-                if (kok) {
-                    const int b = (int)(v / S);
-                    const int vs = (int)(v - (long)b * S);
-                    const int x = vs % g.nx, y = (vs / g.nx) % g.ny, z = vs / (g.nx * g.ny);
-                    bool valid = true;
-                    const int xx = conv_wrap(x + dx, g.nx, g.per[0], valid);
-                    const int yy = conv_wrap(y + dyo, g.ny, g.per[1], valid);
-                    const int zz = conv_wrap(z + dz, g.nz, g.per[2], valid);
-                    if (valid) bv = in[((long)b * S + xx + (long)g.nx * (yy + (long)g.ny * zz)) * g.cin + ci];
-                }
+    for (int t = 0; t < NTW; ++t) {
+        const int k = min(16 * (wv + 4 * t) + row, 27 * CB - 1), tap = k / CB, cl = k % CB;
+        boff[t] = (((tap % 3) * 36 + (tap / 9) * 6 + (tap / 3) % 3) * CB + cl) * 4;
+    }
+    f32x4 acc[NTW][NCO];
+#pragma unroll
+    for (int t = 0; t < NTW; ++t)
+#pragma unroll
+        for (int c = 0; c < NCO; ++c) acc[t][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (long tile = tbeg; tile < tend; ++tile) {
+        const int tb = (int)(tile / ((long)gx * gy * gz)), tr = (int)(tile - (long)tb * gx * gy * gz);
+        const int x0 = 4 * (tr % gx), y0 = 4 * ((tr / gx) % gy), z0 = 4 * (tr / (gx * gy));
+        __syncthreads();
+        for (int e = tid; e < 36 * CB; e += 256) {
+            const int ci = e % CB, hr = e / CB;
+            const int z = z0 + hr / 6 - 1, y = y0 + hr % 6 - 1;
+            bool ok = z <= g.nz && y <= g.ny;
+            const int zz = ok ? conv_wrap(z, g.nz, g.per[2], ok) : 0;
+            const int yy = ok ? conv_wrap(y, g.ny, g.per[1], ok) : 0;
+            const float* src = in + ((long)tb * S + (long)g.nx * (yy + (long)g.ny * zz)) * g.cin + ci0 + ci;
+            unsigned short v[6];
+#pragma unroll
+            for (int q = 0; q < 6; ++q) {
+                const int x = x0 + q - 1;
+                bool okx = ok && x <= g.nx;
+                const int xx = okx ? conv_wrap(x, g.nx, g.per[0], okx) : 0;
+                v[q] = bf16_bits(okx ? src[(long)xx * g.cin] : 0.f);
             }
-            a[i] = __builtin_bit_cast(__bf16, bf16_bits(av));
-            bb[i] = __builtin_bit_cast(__bf16, bf16_bits(bv));
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+                *reinterpret_cast<uint2*>(&xs[c][hr][ci][0]) =
+                    make_uint2(v[c] | ((unsigned)v[c + 1] << 16), v[c + 2] | ((unsigned)v[c + 3] << 16));
         }
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bb, acc, 0, 0, 0);
+        for (int e = tid; e < 8 * CO; e += 256) {
+            const int co = e % CO, o = e / CO;
+            unsigned w[4];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const int x = x0 + (q & 3), y = y0 + 2 * (o & 1) + (q >> 2), z = z0 + (o >> 1);
+                float f = 0.f;
+                if (x < g.nx && y < g.ny && z < g.nz)
+                    f = dy[((long)tb * S + x + (long)g.nx * (y + (long)g.ny * z)) * g.cout + co0 + co];
+                const unsigned h = bf16_bits(f);
+                if (q & 1) w[q >> 1] |= h << 16;
+                else w[q >> 1] = h;
+            }
+            *reinterpret_cast<uint4*>(&ys[o][co][0]) = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            // voxels 32 s + 8 kq + i: octet 4 s + kq, halo rows (z, y) and (z, y + 1)
+            bf16x8 a[NCO];
+#pragma unroll
+            for (int c = 0; c < NCO; ++c)
+                a[c] = *reinterpret_cast<const bf16x8*>(&ys[4 * s + kq][16 * c + row][0]);
+            const unsigned short* xr = &xs[0][0][0][0] + ((2 * s + (kq >> 1)) * 6 + 2 * (kq & 1)) * CB * 4;
+#pragma unroll
+            for (int t = 0; t < NTW; ++t) {
+                const uint2 lo = *reinterpret_cast<const uint2*>(xr + boff[t]);
+                const uint2 hi = *reinterpret_cast<const uint2*>(xr + boff[t] + CB * 4);
+                const uint4 p = make_uint4(lo.x, lo.y, hi.x, hi.y);
+                const bf16x8 b = __builtin_bit_cast(bf16x8, p);
+#pragma unroll
+                for (int c = 0; c < NCO; ++c)
+                    acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[c], b, acc[t][c], 0, 0, 0);
+            }
+        }
     }
     // D[row = co offset 4*kq + j][col = k offset row]
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int co = co0 + 4 * kq + j;
-        const int kc = kk0 + row;
-        if (kc < K) part[((long)chunk * g.cout + co) * g.kp + kc] = acc[j];
+    for (int t = 0; t < NTW; ++t) {
+        const int k = 16 * (wv + 4 * t) + row;
+        if (k >= 27 * CB) continue;
+        const int kg = (k / CB) * g.cin + ci0 + k % CB;
+#pragma unroll
+        for (int c = 0; c < NCO; ++c)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                part[((long)chunk * g.cout + co0 + 16 * c + 4 * kq + j) * g.kp + kg] = acc[t][c][j];
     }
 }
 
-// dW[co][k] += sum over chunks c (in order) of part[c][co][k], k < K (row stride ldw)
-static __global__ void __launch_bounds__(256) conv3d_dw_reduce_kernel(const float* __restrict__ part,
+// dW[co][k] += sum over chunks c of part[c][co][k], k < K (row stride ldw): 64
+// outputs per workgroup, 8 chunk ranges each in order, then the ranges in
+// order (one thread over all chunks took 40 us per layer: too few loads in flight)
+static __global__ void __launch_bounds__(512) conv3d_dw_reduce_kernel(const float* __restrict__ part,
                                                                      int nchunk, int cout, int kp, int K,
                                                                      float* __restrict__ dw, int ldw) {
-    const long id = (long)blockIdx.x * 256 + threadIdx.x;
-    if (id >= (long)cout * K) return;
-    const int co = (int)(id / K), k = (int)(id - (long)co * K);
+    __shared__ float red[8][64];
+    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+    const long id = (long)blockIdx.x * 64 + tx;
+    const bool ok = id < (long)cout * K;
+    const int co = ok ? (int)(id / K) : 0, k = ok ? (int)(id - (long)co * K) : 0;
     float s = 0.f;
-    for (int c = 0; c < nchunk; ++c) s += part[((long)c * cout + co) * kp + k];
-    dw[(long)co * ldw + k] += s;
+    const int c0 = (int)((long)nchunk * ty / 8), c1 = (int)((long)nchunk * (ty + 1) / 8);
+#pragma unroll 8
+    for (int c = c0; c < c1; ++c) s += part[((long)c * cout + co) * kp + k];
+    red[ty][tx] = s;
+    __syncthreads();
+    if (ty == 0 && ok) {
+#pragma unroll
+        for (int r = 1; r < 8; ++r) s += red[r][tx];
+        dw[(long)co * ldw + k] += s;
+    }
 }
 
-// out[i] += sum over parts p (in order) of part[p n + i]
+// out[i] += sum over parts p of part[p n + i], one workgroup per output: each
+// thread every 256th part in order, then a fixed tree (one thread per output
+// over up to 1024 dependent loads took 172 us)
 static __global__ void __launch_bounds__(256) sum_parts_kernel(const float* __restrict__ part, int nparts,
                                                               int n, float* __restrict__ out) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
+    __shared__ float red[256];
+    const int i = blockIdx.x;
     float s = 0.f;
-    for (int p = 0; p < nparts; ++p) s += part[(long)p * n + i];
-    out[i] += s;
+    for (int p = threadIdx.x; p < nparts; p += 256) s += part[(long)p * n + i];
+    red[threadIdx.x] = s;
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+        if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) out[i] += red[0];
 }
 
-// voxels per weight-gradient wave: enough waves to fill the GPU, at least 512
-// voxels each, a multiple of the 32 voxels of one MFMA step
-inline long conv_dw_chunk(const ConvGeom& cg) {
-    const long nvox = (long)cg.nx * cg.ny * cg.nz * cg.batch;
-    const int tiles = (cg.kp / 16) * (cg.cout / 16);
-    const long chunk = std::max<long>(512, (nvox * tiles) / (256L * 64));
-    return (chunk + 31) / 32 * 32;
+// channels of a weight-gradient workgroup: 32 in x 32 out where they divide
+// (108 accumulator registers), else 16 or 8
+inline int conv_dw_cb(const ConvGeom& cg) { return cg.cin % 32 == 0 ? 32 : (cg.cin % 16 == 0 ? 16 : 8); }
+inline int conv_dw_co(const ConvGeom& cg) { return cg.cout % 32 == 0 ? 32 : 16; }
+
+// voxel ranges of the weight gradient: about 768 workgroups (3 per CU), at
+// least one 4 x 4 x 4 tile each
+inline int conv_dw_chunks(const ConvGeom& cg) {
+    const long ntile = (long)((cg.nx + 3) / 4) * ((cg.ny + 3) / 4) * ((cg.nz + 3) / 4) * cg.batch;
+    const long blocks = (long)(cg.cin / conv_dw_cb(cg)) * (cg.cout / conv_dw_co(cg));
+    return (int)std::max<long>(1, std::min<long>(ntile, 768 / blocks));
 }
 
 // floats of workspace conv_dw_launch needs
 inline size_t conv_dw_workspace(const ConvGeom& cg) {
-    const long nvox = (long)cg.nx * cg.ny * cg.nz * cg.batch;
-    const long chunk = conv_dw_chunk(cg);
-    return (size_t)((nvox + chunk - 1) / chunk) * cg.cout * cg.kp;
+    return (size_t)conv_dw_chunks(cg) * cg.cout * cg.kp;
 }
 
 // dW[co][k] += dL/dW of the convolution (row stride ldw), through the per-chunk
 // partials in ws (conv_dw_workspace floats)
 inline void conv_dw_launch(const ConvGeom& cg, const float* in, const float* dy, float* dw, int ldw,
                            float* ws, hipStream_t s) {
-    const long nvox = (long)cg.nx * cg.ny * cg.nz * cg.batch;
-    const int tiles = (cg.kp / 16) * (cg.cout / 16);
-    const long chunk = conv_dw_chunk(cg);
-    const long nchunk = (nvox + chunk - 1) / chunk;
-    conv3d_dw_kernel<<<(unsigned)(tiles * nchunk), 64, 0, s>>>(cg, in, dy, ws, (int)chunk);
+    const int cb = conv_dw_cb(cg), co = conv_dw_co(cg), nchunk = conv_dw_chunks(cg);
+    const int gx = (cg.nx + 3) / 4, gy = (cg.ny + 3) / 4, gz = (cg.nz + 3) / 4;
+    const unsigned nb = (unsigned)((cg.cin / cb) * (cg.cout / co) * nchunk);
+#define MGX_CONV_DW(CB, NCO) conv3d_dw_kernel<CB, NCO><<<nb, 256, 0, s>>>(cg, in, dy, ws, nchunk, gx, gy, gz)
+    if (co == 32) {
+        if (cb == 32) MGX_CONV_DW(32, 2);
+        else if (cb == 16) MGX_CONV_DW(16, 2);
+        else MGX_CONV_DW(8, 2);
+    } else {
+        if (cb == 32) MGX_CONV_DW(32, 1);
+        else if (cb == 16) MGX_CONV_DW(16, 1);
+        else MGX_CONV_DW(8, 1);
+    }
+#undef MGX_CONV_DW
     const long n = (long)cg.cout * 27 * cg.cin;
-    conv3d_dw_reduce_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(ws, (int)nchunk, cg.cout, cg.kp,
-                                                                       27 * cg.cin, dw, ldw);
+    conv3d_dw_reduce_kernel<<<(unsigned)((n + 63) / 64), 512, 0, s>>>(ws, nchunk, cg.cout, cg.kp,
+                                                                     27 * cg.cin, dw, ldw);
 }
 
 // bias gradient, per block: part[block][c] = sum over the block's voxels of
@@ -488,7 +573,7 @@ inline int bias_grad_blocks(long nvox, int c) { return (int)std::min<long>(1024,
 inline void bias_grad_launch(const float* dy, long nvox, int c, float* db, float* ws, hipStream_t s) {
     const int nb = bias_grad_blocks(nvox, c);
     bias_grad_kernel<<<nb, 256, 0, s>>>(dy, nvox, c, ws);
-    sum_parts_kernel<<<(unsigned)((c + 255) / 256), 256, 0, s>>>(ws, nb, c, db);
+    sum_parts_kernel<<<(unsigned)c, 256, 0, s>>>(ws, nb, c, db);
 }
 
 // Data-gradient weights: Wt[ci][tap'*Cout + co] = W[co][(26 - tap')*Cin + ci]
