@@ -277,7 +277,8 @@ MGX_API int mgx_mac_set_options(mgx_mac h, const mgx_mlmg_opts* o) {
     return guarded(h->ctx, [&] {
         MGOpts m;
         to_opts(o, m);
-        const bool relevel = m.max_coarsening_level != h->opts.max_coarsening_level;
+        const bool relevel = m.max_coarsening_level != h->opts.max_coarsening_level ||
+                             deep_levels(m) != deep_levels(h->opts);
         h->opts = m;
         if (relevel) h->dirty = true;
         else h->solver.opts = h->opts;

@@ -259,7 +259,7 @@ void MacSolver::setup(const MacGeom& g, const MGOpts& o) {
                            g.per[0] == g0.per[0] && g.per[1] == g0.per[1] && g.per[2] == g0.per[2];
     g0 = g;
     opts = o;
-    nlev = mac_nlevels(g, o.max_coarsening_level, deep);
+    nlev = mac_nlevels(g, o.max_coarsening_level, deep && deep_levels(o));
     for (int d = 0; d < 3; ++d) beta0[d].alloc(g.nface(d) * sizeof(double));
     const long n = g.ncell();
     if (g.has_a) acoef0.alloc(n * sizeof(double));
@@ -282,7 +282,7 @@ void MacSolver::setup(const MacGeom& g, const MGOpts& o) {
 
 void MacSolver::set_deep(bool on) {
     deep = on;
-    nlev = mac_nlevels(g0, opts.max_coarsening_level, deep);
+    nlev = mac_nlevels(g0, opts.max_coarsening_level, deep && deep_levels(opts));
 }
 
 void MacSolver::set_robin(int d, int side, std::vector<double> a, std::vector<double> b) {

@@ -720,7 +720,7 @@ void NodalSolver::setup(const NodalGeom& g, const MGOpts& o) {
                             g.per[2] == g0.per[2];
     g0 = g;
     opts = o;
-    nlev = nodal_nlevels(g, o.max_coarsening_level, true);
+    nlev = nodal_nlevels(g, o.max_coarsening_level, deep_levels(o));
     const long nn = g.nnode();
     sig0_buf.alloc(g.nsig() * sizeof(double));
     if (!keep_sigma) MGX_HIP(hipMemset(sig0_buf.p, 0, g.nsig() * sizeof(double)));

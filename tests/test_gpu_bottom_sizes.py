@@ -151,3 +151,25 @@ def test_eb_bottom_of_every_size(ctx, orc, levels):
     assert info.converged and info.nlevels == levels + 1
     r = np.where(mask, b - orc.eb_nodal_apply(g, ct, mom, sigma, x), 0.0)
     assert np.max(np.abs(r)) <= 2 * RTOL * np.max(np.abs(b))
+
+
+# levels of 2 and 3 cells are made only with four sweeps or more per cycle:
+# with fewer the cycle did not converge through them (49 cycles without)
+@pytest.mark.parametrize("nu1,nu2", [(0, 1), (1, 0), (1, 2), (2, 2)])
+def test_mac_few_sweeps_converge(ctx, nu1, nu2):
+    from incflo_amd import mgx
+    n = (36, 20, 12)
+    _say(f"case mac {n} nu {nu1},{nu2}")
+    ph = tuple(m / 20 for m in n)
+    rng = np.random.default_rng(7)
+    beta = [0.5 + rng.random((n[2] + (d == 2), n[1] + (d == 1), n[0] + (d == 0))) for d in range(3)]
+    b = rng.standard_normal((n[2], n[1], n[0]))
+    bxs = B.chop_domain(n, 64)
+    P = mgx.MacProjector(ctx, mgx.make_level(n, bxs, periodic=(0, 0, 0), prob_hi=ph))
+    P.setDomainBC((D, N, N), (N, D, N))
+    P.set_options(mgx.default_opts(nu1=nu1, nu2=nu2, maxiter=200))
+    P.set_beta(*[ctx.array(B.faces_to_boxed(beta[d], bxs, 0, d)) for d in range(3)], ng=0)
+    xd = ctx.array(B.field_size(bxs, 0, 1))
+    info = P.solve(xd, 0, ctx.array(B.to_boxed(b, bxs, 0)), 0, RTOL)
+    P.close()
+    assert info.converged and info.vcycles <= 60
