@@ -56,11 +56,12 @@ struct MacLevel {
     MacGeom g;
     MGeomK kg;
     MCoef<T> c;
-    DevBuf beta_buf[3], a_buf, b_buf, x_buf, r_buf;
+    DevBuf beta_buf[3], a_buf, b_buf, x_buf, x2_buf, r_buf;
     T* beta[3] = {nullptr, nullptr, nullptr};
     T* a = nullptr;  // Helmholtz cell coefficient (null: none)
     T* b = nullptr;
     T* x = nullptr;
+    T* x2 = nullptr;  // the iterate between the down and the up leg
     T* r = nullptr;
 };
 

@@ -9,6 +9,7 @@
 #include <cstring>
 
 #include "mac_mg.h"
+#include "mac_tile_kernels.h"
 #include "mgx_ctx.h"
 
 namespace mgx {
@@ -48,9 +49,13 @@ void MacHierarchy<T>::build(const MacGeom& g0, int nlev) {
         }
         if (l > 0) lv.b_buf.alloc(n * sizeof(T));
         lv.x_buf.alloc(n * sizeof(T));
-        if (l < nlev - 1) lv.r_buf.alloc(n * sizeof(T));
+        if (l < nlev - 1) {
+            lv.x2_buf.alloc(n * sizeof(T));
+            lv.r_buf.alloc(n * sizeof(T));
+        }
         lv.b = lv.b_buf.template as<T>();
         lv.x = lv.x_buf.template as<T>();
+        lv.x2 = lv.x2_buf.template as<T>();
         lv.r = lv.r_buf.template as<T>();
     }
     bottom_work.alloc(bottom_work_doubles(L.back().g.ncell(), 7) * sizeof(double));
@@ -98,11 +103,21 @@ void MacHierarchy<T>::set_acoef(const double* a0, hipStream_t s) {
     }
 }
 
+// the level's part of the tile kernels' arguments (w: the level below, or v)
 template <class T>
-static void gsrb(MacLevel<T>& lv, hipStream_t s) {
-    for (int color = 0; color < 2; ++color)
-        mac_gsrb_kernel<T><<<grid3((lv.g.n[0] + 1) / 2, lv.g.n[1], lv.g.n[2]), block3(), 0, s>>>(
-            lv.kg, lv.c, lv.beta[0], lv.beta[1], lv.beta[2], lv.a, lv.b, lv.x, color);
+static MacTileArgs<T> mac_tile_args(const MacLevel<T>& v, const MacLevel<T>& w) {
+    MacTileArgs<T> a{};
+    a.g = v.kg;
+    a.gc = w.kg;
+    a.c = v.c;
+    a.bx = v.beta[0];
+    a.by = v.beta[1];
+    a.bz = v.beta[2];
+    a.a = v.a;
+    a.b = v.b;
+    a.bc = w.b;
+    a.xc = w.x;
+    return a;
 }
 
 // the options a V-cycle's launches depend on
@@ -202,18 +217,10 @@ void MacHierarchy<T>::vcycle_body(const MGOpts& o, hipStream_t s, int* bottom_it
     const int nl = (int)L.size();
     // levels lc..nl-2 in one workgroup (lc == nl - 1: none)
     const int lc = mac_coarse_first(L);
-    for (int l = 0; l < lc; ++l) {
-        MacLevel<T>& lv = L[l];
-        const long n = lv.g.ncell();
-        if (l > 0 || !x0_guess) zero_kernel<T><<<grid1d(n), 256, 0, s>>>(lv.x, n);
-        for (int q = 0; q < o.nu1; ++q) gsrb(lv, s);
-        mac_resid_kernel<T, T, MK_RESID><<<grid3(lv.g.n[0], lv.g.n[1], lv.g.n[2]), block3(), 0, s>>>(
-            lv.kg, lv.c, lv.beta[0], lv.beta[1], lv.beta[2], lv.a, lv.b, lv.x, nullptr, nullptr,
-            lv.r, nullptr);
-        MacLevel<T>& cv = L[l + 1];
-        mac_restrict_kernel<T><<<grid3(cv.g.n[0], cv.g.n[1], cv.g.n[2]), block3(), 0, s>>>(
-            lv.kg, cv.kg, lv.r, cv.b);
-    }
+    // down: x (a guess on level 0) -> x2; up: x2 -> x
+    for (int l = 0; l < lc; ++l)
+        mac_tile_sweeps(mac_tile_args(L[l], L[l + 1]), l == 0 && x0_guess ? MT_X : MT_ZERO, L[l].x, L[l].x2,
+                        o.nu1, true, s);
     if (lc < nl - 1) mac_coarse_cycle_kernel<T><<<1, 1024, 0, s>>>(mac_coarse_args(L, lc, o, 0));
     {
         MacLevel<T>& lb = L[nl - 1];
@@ -229,12 +236,8 @@ void MacHierarchy<T>::vcycle_body(const MGOpts& o, hipStream_t s, int* bottom_it
     }
     x0_guess = false;
     if (lc < nl - 1) mac_coarse_cycle_kernel<T><<<1, 1024, 0, s>>>(mac_coarse_args(L, lc, o, 1));
-    for (int l = lc - 1; l >= 0; --l) {
-        MacLevel<T>& lv = L[l];
-        mac_prolong_add_kernel<T><<<grid3(lv.g.n[0], lv.g.n[1], lv.g.n[2]), block3(), 0, s>>>(
-            lv.kg, L[l + 1].kg, L[l + 1].x, lv.x);
-        for (int q = 0; q < o.nu2; ++q) gsrb(lv, s);
-    }
+    for (int l = lc - 1; l >= 0; --l)
+        mac_tile_sweeps(mac_tile_args(L[l], L[l + 1]), MT_PROLONG, L[l].x2, L[l].x, o.nu2, false, s);
 }
 
 template class MacHierarchy<double>;

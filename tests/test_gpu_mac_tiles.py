@@ -1,0 +1,67 @@
+"""GPU test of the cell-centred V-cycle's tile kernels at the level sizes where
+the tile changes (register tiles up to 131072 cells, 8 x 8 x 8 up to 400000,
+16 x 16 x 8 above) with ragged last tiles, periodic and bounded sides, sweep
+counts that need no launch, one or several per leg, FP64 and mixed.
+
+The check is the answer's residual under the oracle's FP64 operator: the solve
+stops at rtol in the library's operator and the two round differently by a few
+eps per row, below rtol here, so 2 rtol bounds it."""
+import numpy as np
+import pytest
+
+from incflo_amd import boxes as B
+
+pytestmark = pytest.mark.gpu
+
+D, N = 1, 2
+RTOL = 1e-10
+CASES = [  # cells, periodic, lo, hi, nu1, nu2, mixed
+    ((36, 20, 12), (1, 0, 1), (0, N, 0), (0, D, 0), 2, 2, False),
+    ((36, 20, 12), (0, 1, 0), (N, 0, D), (D, 0, N), 0, 1, False),
+    ((36, 20, 12), (1, 1, 1), (0, 0, 0), (0, 0, 0), 3, 0, False),
+    ((20, 36, 12), (0, 0, 0), (N, N, N), (N, N, N), 1, 4, True),
+    ((100, 44, 36), (0, 1, 1), (D, 0, 0), (N, 0, 0), 2, 2, False),    # 158400 cells
+    ((100, 44, 36), (1, 1, 1), (0, 0, 0), (0, 0, 0), 2, 2, True),
+    ((108, 76, 60), (0, 0, 1), (N, D, 0), (N, N, 0), 2, 2, False),    # 492480 cells
+    ((108, 76, 60), (1, 1, 0), (0, 0, N), (0, 0, D), 2, 2, True),
+]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from incflo_amd import mgx
+    c = mgx.Context(0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("n,per,bclo,bchi,nu1,nu2,mixed", CASES)
+def test_mac_tile_legs(ctx, orc, n, per, bclo, bchi, nu1, nu2, mixed):
+    from incflo_amd import mgx
+    print(f"case mac tiles {n} nu {nu1},{nu2} mixed {mixed}", flush=True)
+    h = 1.0 / n[1]
+    ph = tuple(m * h for m in n)
+    g = orc.Geom.make(n, periodic=per, bclo=bclo, bchi=bchi, prob_hi=ph)
+    rng = np.random.default_rng(sum(n) + nu1)
+    beta = [0.5 + rng.random(orc.face_shape(g, d)) for d in range(3)]
+    for d in range(3):
+        if per[d]:
+            lo, hi = [slice(None)] * 3, [slice(None)] * 3
+            lo[2 - d], hi[2 - d] = 0, -1
+            beta[d][tuple(hi)] = beta[d][tuple(lo)]
+    b = rng.standard_normal(g.cell_shape())
+    if all(per[d] or (bclo[d] != D and bchi[d] != D) for d in range(3)):
+        b -= b.mean()
+    bxs = B.chop_domain(n, 64)
+    P = mgx.MacProjector(ctx, mgx.make_level(n, bxs, periodic=per, prob_hi=ph))
+    P.setDomainBC(bclo, bchi)
+    P.set_options(mgx.default_opts(nu1=nu1, nu2=nu2, maxiter=200, bottom_maxiter=200))
+    P.set_beta(*[ctx.array(B.faces_to_boxed(beta[d], bxs, 0, d)) for d in range(3)], ng=0)
+    rd = ctx.array(B.to_boxed(b, bxs, 0, periodic=per))
+    xd = ctx.array(B.field_size(bxs, 0, 1))
+    info = P.solve(xd, 0, rd, 0, RTOL, mode=mgx.MODE_MIXED if mixed else mgx.MODE_FP64)
+    x = B.from_boxed(xd.download(), bxs, 0, g.cell_shape())
+    P.close()
+    assert info.converged and info.nlevels > 1
+    r = orc.mac_residual(g, beta, b, x)
+    assert np.max(np.abs(r)) <= 2 * RTOL * np.max(np.abs(b))
