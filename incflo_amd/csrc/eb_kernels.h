@@ -29,19 +29,6 @@ struct EBLev {
     const unsigned char* mask;  // per node: 1 active
 };
 
-enum { EB_APPLY = 0, EB_RESID = 1, EB_JACOBI = 2, EB_UPDRES = 3 };
-
-struct EBArgs {
-    EBLev L;
-    const double* x;
-    const double* cor;   // EB_UPDRES: x + cor is the new iterate
-    const double* b;
-    double* xout;
-    double* rout;
-    unsigned long long* norm;
-    double omega;
-};
-
 // wrapped cell index along d of node i's side a; -1 outside a non-periodic domain
 __device__ __forceinline__ int eb_cell(const KGeom& g, int d, int i, int a) {
     int c = i - 1 + a;
@@ -54,11 +41,10 @@ __device__ __forceinline__ int eb_node(const KGeom& g, int d, int i) {
     return i;
 }
 
-// (L x)_n and the diagonal of L at node (i, j, k); x + cor when cor != nullptr
-__device__ inline double eb_apply_node(const EBLev& L, const double* x, const double* cor, int i,
-                                       int j, int k, double& diag) {
+// (L x)_n at node (i, j, k)
+__device__ inline double eb_apply_node(const EBLev& L, const double* x, int i, int j, int k) {
     const KGeom& g = L.g;
-    double acc = 0.0, dg = 0.0;
+    double acc = 0.0;
     for (int a = 0; a < 8; ++a) {
         const int ax = a & 1, ay = (a >> 1) & 1, az = (a >> 2) & 1;
         const int c0 = eb_cell(g, 0, i, ax), c1 = eb_cell(g, 1, j, ay), c2 = eb_cell(g, 2, k, az);
@@ -82,18 +68,14 @@ __device__ inline double eb_apply_node(const EBLev& L, const double* x, const do
             const int mj = eb_node(g, 1, j - 1 + ay + ((m >> 1) & 1));
             const int mk = eb_node(g, 2, k - 1 + az + ((m >> 2) & 1));
             const long mid = mi + (long)g.nn[0] * (mj + (long)g.nn[1] * mk);
-            double v = x[mid];
-            if (cor) v += cor[mid];
-            e += Kr[p * 8 + m] * v;
+            e += Kr[p * 8 + m] * x[mid];
         }
         acc -= s * e;
-        dg -= s * Kr[p * 9];
     }
-    diag = dg;
     return acc;
 }
 
-// The rows of the EB operator for the bottom solve: inactive nodes are held at zero.
+// The rows of the EB operator, for the row tables and the bottom solve: inactive nodes are held at zero.
 struct EBRows {
     static constexpr int NS = 27;
     static constexpr bool kRedBlack = false;
@@ -124,41 +106,160 @@ struct EBRows {
 };
 MGX_BOTTOM_INSTANCE(extern, EBRows, double);
 
-static __global__ void __launch_bounds__(256) eb_stencil_kernel(EBArgs a, int mode) {
+// The operator alone (mgx_nodal_apply): out = L x, 0 on inactive nodes.
+static __global__ void __launch_bounds__(256) eb_apply_kernel(EBLev L, const double* __restrict__ x,
+                                                              double* __restrict__ out) {
     int i, j, k;
-    const bool valid = grid_point(a.L.g.nn[0], a.L.g.nn[1], i, j, k);
-    double r = 0.0;
-    if (valid) {
-        const long id = i + (long)a.L.g.nn[0] * (j + (long)a.L.g.nn[1] * k);
-        if (a.L.mask[id]) {
-            double dg;
-            const double lx =
-                eb_apply_node(a.L, a.x, mode == EB_UPDRES ? a.cor : nullptr, i, j, k, dg);
-            if (mode == EB_APPLY) {
-                a.xout[id] = lx;
-            } else if (mode == EB_JACOBI) {
-                a.xout[id] = (dg != 0.0) ? a.x[id] + a.omega * (a.b[id] - lx) / dg : 0.0;
-            } else {
-                r = a.b[id] - lx;
-                a.rout[id] = r;
-                if (mode == EB_UPDRES) a.xout[id] = a.x[id] + a.cor[id];
-            }
-        } else if (mode == EB_APPLY || mode == EB_JACOBI) {
-            a.xout[id] = 0.0;
+    if (!grid_point(L.g.nn[0], L.g.nn[1], i, j, k)) return;
+    const long id = i + (long)L.g.nn[0] * (j + (long)L.g.nn[1] * k);
+    out[id] = L.mask[id] ? eb_apply_node(L, x, i, j, k) : 0.0;
+}
+
+// ---- the solver's passes over assembled rows --------------------------------
+// Going through the cells of a node costs 8 dependent look-ups (cell class,
+// then sigma or the cut element) and 64 loads of x, of which 37 are repeats:
+// 84 us for a residual or sweep of 257 x 65 x 64 nodes, whose data take 8 us.
+// The rows of the nodes at cut cells are therefore assembled once per sigma
+// (27 coefficients, one array per neighbour, so every load is coalesced over
+// the rows); the other active nodes see regular cells only and are swept by
+// the plain nodal stencil kernel, with the nodes listed here as type 2.  A
+// level of at most kEBRowNodes nodes has all its rows in the table and takes
+// one launch per pass: below that size the two launches of the split cost
+// more than reading the 27 coefficients.
+struct EBRowArgs {
+    KGeom g;
+    const int* ids;      // node of each row; nullptr: row r is node r
+    int nrow;
+    const double* C;     // 27 x nrow, coefficient of neighbour (ox, oy, oz) at ox + 3 oy + 9 oz
+    const double* x;
+    const double* cor;   // KS_UPDRES: x + cor is the new iterate
+    const double* b;
+    double* xout;
+    double* rout;
+    unsigned long long* norm;
+    double* x1out;       // KS_RESID / KS_UPDRES, optional: first Jacobi iterate from zero for r
+    double omega;
+};
+
+static __global__ void __launch_bounds__(256) eb_rows_build_kernel(EBLev L, const int* __restrict__ ids,
+                                                                   int nrow, double* __restrict__ C) {
+    const int r = blockIdx.x * 256 + threadIdx.x;
+    if (r >= nrow) return;
+    const int id = ids ? ids[r] : r;
+    const int j0 = id / L.g.nn[0], i = id - j0 * L.g.nn[0], k = j0 / L.g.nn[1], j = j0 - k * L.g.nn[1];
+    double c[27];
+    const bool act = EBRows{L}.row(id, i, j, k, c);
+#pragma unroll
+    for (int s = 0; s < 27; ++s) C[(long)s * nrow + r] = act ? c[s] : 0.0;
+}
+
+// One thread per row, one wave per workgroup (the small levels have too few
+// rows to fill the card with larger ones).  Bound by load latency: the wave
+// limit lets the compiler keep all 54 loads of a row in flight (left to itself
+// it took 25 registers and made the residual pass 1.6 times a sweep).
+// Inactive rows are zero rows with b = x = 0, so they need no test.
+template <int MODE>
+static __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 4))) eb_rows_kernel(EBRowArgs a) {
+    const int r = blockIdx.x * 64 + threadIdx.x;
+    double res = 0.0;
+    if (r < a.nrow) {
+        const KGeom& g = a.g;
+        const int id = a.ids ? a.ids[r] : r;
+        const double* C = a.C + r;
+        const long nr = a.nrow;
+        const double dg = C[13 * nr];
+        if (MODE == KS_JFIRST) {
+            a.xout[id] = dg != 0.0 ? a.omega * a.b[id] / dg : 0.0;
         } else {
-            a.rout[id] = 0.0;
-            if (mode == EB_UPDRES) a.xout[id] = 0.0;
+            const int j0 = id / g.nn[0], n3[3] = {id - j0 * g.nn[0], j0 % g.nn[1], j0 / g.nn[1]};
+            // neighbours beyond a non-periodic side have coefficient 0: any index will do
+            int o[3][3];
+            int stride = 1;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                const int m = n3[d], n = g.nn[d];
+                o[d][0] = stride * (m > 0 ? m - 1 : (g.per[d] ? n - 1 : 0));
+                o[d][1] = stride * m;
+                o[d][2] = stride * (m < n - 1 ? m + 1 : (g.per[d] ? 0 : m));
+                stride *= n;
+            }
+            double acc = 0.0, v[27], w[27];
+#pragma unroll
+            for (int s = 0; s < 27; ++s) {
+                const int e = o[0][s % 3] + o[1][(s / 3) % 3] + o[2][s / 9];
+                v[s] = a.x[e];
+                if (MODE == KS_UPDRES) w[s] = a.cor[e];
+            }
+            __builtin_amdgcn_sched_barrier(0);  // all loads of x before their uses
+#pragma unroll
+            for (int s = 0; s < 27; ++s) {
+                if (MODE == KS_UPDRES) v[s] += w[s];
+                acc += C[s * nr] * v[s];
+            }
+            const double xc = v[13];
+            const double q = a.b[id] - acc;
+            if (MODE == KS_JACOBI) {
+                a.xout[id] = dg != 0.0 ? xc + a.omega * q / dg : 0.0;
+            } else {
+                res = q;
+                a.rout[id] = q;
+                if (MODE == KS_UPDRES) a.xout[id] = xc;
+                if (a.x1out) a.x1out[id] = dg != 0.0 ? a.omega * q / dg : 0.0;
+            }
         }
     }
-    if ((mode == EB_RESID || mode == EB_UPDRES) && a.norm) {
+    if ((MODE == KS_RESID || MODE == KS_UPDRES) && a.norm) {
         // one atomic per wave; every lane stays active through the shuffles
-        double v = nabs(r);
+        double v = nabs(res);
         for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
-        if ((threadIdx.x & 63) == 0) atomic_max_nonneg(a.norm, v);
+        if (threadIdx.x == 0) atomic_max_nonneg(a.norm, v);
     }
 }
 
-// x = 0 on inactive nodes (after prolongation)
+// Full weighting onto a level with all its rows in the table, with the first
+// Jacobi sweep from zero (diag: the table's centre coefficients).  Residuals
+// of inactive nodes are 0, and a coarse inactive node has only such around it.
+static __global__ void __launch_bounds__(64) eb_restrict_kernel(KGeom gf, KGeom gc,
+                                                                const double* __restrict__ rf,
+                                                                double* __restrict__ rc,
+                                                                const double* __restrict__ diag,
+                                                                double omega, double* __restrict__ x1) {
+    const int id = blockIdx.x * 64 + threadIdx.x;
+    if (id >= gc.nn[0] * gc.nn[1] * gc.nn[2]) return;
+    const int j0 = id / gc.nn[0], n3[3] = {id - j0 * gc.nn[0], j0 % gc.nn[1], j0 / gc.nn[1]};
+    int o[3][3];
+    double w[3][3];
+    int stride = 1;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            int f = 2 * n3[d] + q - 1;
+            w[d][q] = q == 1 ? 0.5 : 0.25;
+            if (gf.per[d]) {
+                f = f < 0 ? f + gf.nn[d] : (f >= gf.nn[d] ? f - gf.nn[d] : f);
+            } else if (f < 0 || f >= gf.nn[d]) {
+                w[d][q] = 0.0;
+                f = 2 * n3[d];
+            }
+            o[d][q] = stride * f;
+        }
+        stride *= gf.nn[d];
+    }
+    double acc = 0.0;
+#pragma unroll
+    for (int s = 0; s < 27; ++s)
+        acc += w[0][s % 3] * w[1][(s / 3) % 3] * w[2][s / 9] *
+               rf[o[0][s % 3] + o[1][(s / 3) % 3] + o[2][s / 9]];
+    if (is_dir(gc, n3[0], n3[1], n3[2])) acc = 0.0;
+    rc[id] = acc;
+    if (x1) {
+        const double dg = diag[id];
+        x1[id] = dg != 0.0 ? omega * acc / dg : 0.0;
+    }
+}
+
+// x = 0 on inactive nodes
 static __global__ void eb_mask_kernel(const unsigned char* __restrict__ mask, double* __restrict__ x,
                                       long n) {
     const long id = (long)blockIdx.x * blockDim.x + threadIdx.x;

@@ -44,6 +44,14 @@ struct EBLevelData {
     std::vector<unsigned char> mask_h;
     DevBuf cidx, cutc, child, mask, K, Egeom, W, V;
     DevBuf sig_buf, b_buf, x_buf, x2_buf, r_buf;
+    // assembled rows: of every node (ids empty), or of the active nodes at
+    // cells that are not regular, the others (type 1) being swept by the plain
+    // stencil kernel
+    DevBuf rows, ids, types;
+    int nrow = 0;
+    bool all_rows = true;
+    double* x = nullptr;   // iterate and the sweeps' other buffer (they swap)
+    double* x2 = nullptr;
     double E[64];
     int ncut = 0;
 };
@@ -70,8 +78,11 @@ class EBNodal {
     const double* sig0 = nullptr;
 
    private:
-    void vcycle(const MGOpts& o, hipStream_t s);
-    void smooth(int l, int sweeps, bool from_zero, const MGOpts& o, hipStream_t s);
+    // first: level 0's first sweep has been made by the residual pass
+    void vcycle(const MGOpts& o, bool first, hipStream_t s);
+    void smooth(int l, int sweeps, bool from_zero, bool first, const MGOpts& o, hipStream_t s);
+    template <int MODE>
+    void pass(int l, EBRowArgs a, hipStream_t s);
 };
 
 }  // namespace mgx

@@ -531,14 +531,10 @@ MGX_API int mgx_nodal_apply(mgx_nodal h, const double* phi, int phi_ng, double* 
             kg, h->layout.dev_boxes(), h->layout.tiles(REG_NODE), phi, phi_ng, h->rhs.as<double>());
         if (h->eb) {
             h->eb->set_sigma(h->solver.sigma0(), h->stream());
-            EBArgs e{};
-            e.L = h->eb->lev(0);
-            e.x = h->rhs.as<double>();
-            e.xout = h->solver.phi;
             eb_mask_kernel<<<grid1d(h->g.nnode()), 256, 0, h->stream()>>>(
                 h->eb->mask0(), h->rhs.as<double>(), h->g.nnode());
-            eb_stencil_kernel<<<grid3(h->g.nn[0], h->g.nn[1], h->g.nn[2]), block3(), 0,
-                                h->stream()>>>(e, EB_APPLY);
+            eb_apply_kernel<<<grid3(h->g.nn[0], h->g.nn[1], h->g.nn[2]), block3(), 0,
+                              h->stream()>>>(h->eb->lev(0), h->rhs.as<double>(), h->solver.phi);
         } else {
             SArgs<double, double> a{};
             a.g = kg;

@@ -696,6 +696,7 @@ void NodalHierarchy<T>::vcycle_body(const MGOpts& o, hipStream_t s, int* bottom_
 template void launch_stencil<double, double, KS_APPLY>(const NodalGeom&, SArgs<double, double>, hipStream_t, bool, TileSet*);
 template void launch_stencil<double, double, KS_RESID>(const NodalGeom&, SArgs<double, double>, hipStream_t, bool, TileSet*);
 template void launch_stencil<double, double, KS_JACOBI>(const NodalGeom&, SArgs<double, double>, hipStream_t, bool, TileSet*);
+template void launch_stencil<double, double, KS_UPDRES>(const NodalGeom&, SArgs<double, double>, hipStream_t, bool, TileSet*);
 template void launch_stencil<double, double, KS_JFIRST>(const NodalGeom&, SArgs<double, double>, hipStream_t, bool, TileSet*);
 template void launch_stencil<float, float, KS_APPLY>(const NodalGeom&, SArgs<float, float>, hipStream_t, bool, TileSet*);
 template void launch_stencil<float, float, KS_JACOBI>(const NodalGeom&, SArgs<float, float>, hipStream_t, bool, TileSet*);
