@@ -71,14 +71,21 @@ GdArrays bind(mgx_adv_s* h, const double* qg, const double* f, const double* adv
     return a;
 }
 
-void run_stages(mgx_adv_s* h, const GdArrays& a) {
-    const dim3 gc = grid3(h->g.n[0], h->g.n[1], h->g.n[2]);
-    const dim3 gf = grid3(h->g.n[0] + 1, h->g.n[1] + 1, h->g.n[2] + 1), bl = block3();
+template <bool EX, int NC>
+void launch_stages(mgx_adv_s* h, const GdArrays& a) {
+    const dim3 gf = plane_grid(h->g.n[0] + 1, h->g.n[1] + 1, h->g.n[2] + 1);
     hipStream_t s = h->stream();
-    gd_ppm_kernel<<<gc, bl, 0, s>>>(h->g, a);
-    gd_edge_kernel<<<gf, bl, 0, s>>>(h->g, a);
-    gd_trans_kernel<<<gf, bl, 0, s>>>(h->g, a);
-    gd_final_kernel<<<gf, bl, 0, s>>>(h->g, a);
+    gd_ppm_kernel<EX, NC><<<grid3(h->g.n[0], h->g.n[1], h->g.n[2]), block3(), 0, s>>>(h->g, a);
+    gd_edge_kernel<EX, NC><<<gf, 256, 0, s>>>(h->g, a);
+    gd_trans_kernel<EX, NC><<<gf, 256, 0, s>>>(h->g, a);
+    gd_final_kernel<EX, NC><<<gf, 256, 0, s>>>(h->g, a);
+}
+
+void run_stages(mgx_adv_s* h, const GdArrays& a) {
+    if (a.extrap) launch_stages<true, 3>(h, a);
+    else if (a.nc == 1) launch_stages<false, 1>(h, a);
+    else if (a.nc == 2) launch_stages<false, 2>(h, a);
+    else launch_stages<false, 3>(h, a);
 }
 
 // ghosted canonical cells (2 layers) from a boxed field
@@ -241,7 +248,7 @@ MGX_API int mgx_adv_convective_term(mgx_adv h, const double* vel, int vel_ng, co
             h->flbuf.alloc(3 * 3 * h->NF * sizeof(double));
             for (int d = 0; d < 3; ++d) fo.f[d] = h->flbuf.as<double>() + 3 * d * h->NF;
         }
-        gd_conv_kernel<<<grid3(h->g.n[0] + 1, h->g.n[1] + 1, h->g.n[2] + 1), block3(), 0,
+        gd_conv_kernel<<<plane_grid(h->g.n[0] + 1, h->g.n[1] + 1, h->g.n[2] + 1), 256, 0,
                          h->stream()>>>(h->g, a, h->cbuf.as<double>(), fo, 0);
         gd_cells_out_kernel<<<h->layout.ntiles[REG_CELL], 256, 0, h->stream()>>>(
             h->g, h->layout.dev_boxes(), h->layout.tiles(REG_CELL), conv, conv_ng, 3,
@@ -311,7 +318,7 @@ MGX_API int mgx_adv_scalar_term(mgx_adv h, const double* state, int s_ng, int nc
                               force ? h->sfbuf.as<double>() + n0 * N : nullptr,
                               h->abuf.as<double>(), dt, false, nc, cons, bc);
             run_stages(h, a);
-            gd_conv_kernel<<<grid3(h->g.n[0] + 1, h->g.n[1] + 1, h->g.n[2] + 1), block3(), 0,
+            gd_conv_kernel<<<plane_grid(h->g.n[0] + 1, h->g.n[1] + 1, h->g.n[2] + 1), 256, 0,
                              h->stream()>>>(h->g, a, h->cbuf.as<double>(), fo, n0);
             if (want_face)
                 for (int d = 0; d < 3; ++d)
