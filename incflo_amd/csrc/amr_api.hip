@@ -482,9 +482,8 @@ class AmrNodal {
             // correction below)
             ap.x = e;
             ap.b = nullptr;
+            ap.nmask = ft;  // L e on dF, 0 elsewhere
             launch_stencil<T, T, KS_APPLY>(f.g, ap, s, false, &f.tiles);
-            if (nbk)
-                amr_mask_bdry_kernel<T><<<nbk, tile_block(), 0, s>>>(kf, ft, f.yT.as<T>(), f.yT.as<T>(), tl);
             restrict_full<T>(f.g, gcl, f.yT.as<T>(), w, s);
             if (l == 1) {
                 SArgs<T, T> ac{};

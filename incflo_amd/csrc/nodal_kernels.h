@@ -180,7 +180,8 @@ struct SArgs {
     double omega1;   //   iterate from zero of the next V-cycle (saves its pass)
     // optional node types (composite AMR levels): 1 unknown, 2 fixed (JACOBI
     // keeps the value), 0 outside (JACOBI / JFIRST write 0); RESID writes
-    // r = 0 on every node that is not an unknown
+    // r = 0 on every node that is not an unknown; APPLY writes 0 on every node
+    // that is not fixed
     const unsigned char* nmask;
     // scaled reduced-precision V-cycle (0 means 1): UPDRES adds cor_scale*cor;
     // RESID/UPDRES store rscale*r and x1 from x1scale*r
@@ -319,7 +320,7 @@ static __global__ void __launch_bounds__(TXP == 64 && NPT == 1 ? 512 : 256)
     const KGeom& g = a.g;
     const int tx = threadIdx.x, ty = threadIdx.y, tid = tx + TX * ty;
     const int nb = a.gx * a.gy * a.gz;
-    const int lb = a.tiles ? a.tiles[blockIdx.x] : xcd_remap(blockIdx.x, nb);
+    const int lb = a.tiles ? a.tiles[xcd_remap(blockIdx.x, gridDim.x)] : xcd_remap(blockIdx.x, nb);
     const int bx = lb % a.gx, by = (lb / a.gx) % a.gy, bz = lb / (a.gx * a.gy);
     const int i0 = bx * TX, j0 = by * NY, k0 = bz * a.kz;
     const int k1 = min(k0 + a.kz, g.nn[2]);
@@ -496,7 +497,7 @@ static __global__ void __launch_bounds__(TXP == 64 && NPT == 1 ? 512 : 256)
                         v = c + (bv - acc) * (a.omega * diag_rcp(-a.c.diag4 * ssum));
                     *byte_add(a.xout + kp, oox[n]) = st<T>(v);
                 } else if (MODE == KS_APPLY) {
-                    *byte_add(a.rout + kp, ooc[n]) = st<TC>(acc);
+                    *byte_add(a.rout + kp, ooc[n]) = st<TC>(MASK && nt != 2 ? (TA)0 : acc);
                 } else {
                     const TA r = (dir || nt != 1) ? (TA)0 : (bv - acc);
                     *byte_add(a.rout + kp, ooc[n]) = st<TC>((acc_t<TC>)(rsc * (double)r));
@@ -947,7 +948,7 @@ static __global__ void __launch_bounds__(256) nodal_jacobi_dma_kernel(SArgs<T, T
     const KGeom& g = a.g;
     const int tx = threadIdx.x, ty = threadIdx.y;
     const int nb = a.gx * a.gy * a.gz;
-    const int lb = a.tiles ? a.tiles[blockIdx.x] : xcd_remap(blockIdx.x, nb);
+    const int lb = a.tiles ? a.tiles[xcd_remap(blockIdx.x, gridDim.x)] : xcd_remap(blockIdx.x, nb);
     const int bx = lb % a.gx, by = (lb / a.gx) % a.gy, bz = lb / (a.gx * a.gy);
     const int i0 = bx * TX, j0 = by * NY, k0 = bz * a.kz;
     const int k1 = min(k0 + a.kz, g.nn[2]);
