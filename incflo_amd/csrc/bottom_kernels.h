@@ -646,6 +646,13 @@ __device__ __forceinline__ void bottom_krylov(Plan& pl, const T* b_in, T* x_out,
     block_reduce<1, 1>(rn0, red, phase);
     const double rnorm0 = rn0[0], stop = a.rtol * rnorm0;
 
+    auto passes = [&]() {
+        double u[1] = {0.0};
+#pragma unroll
+        for (int q = 0; q < (NPT ? NPT : cnt); ++q) u[0] = fmax(u[0], unscaled(q));
+        block_reduce<1, 1>(u, red, phase);
+        return u[0] <= stop;
+    };
     // 0: converged, 1: broke down, 2: iteration limit; both from zero
     auto bicgstab = [&](int& iters) -> int {
         double g[1] = {0.0};
@@ -658,7 +665,9 @@ __device__ __forceinline__ void bottom_krylov(Plan& pl, const T* b_in, T* x_out,
         block_reduce<1, 0>(g, red, phase);
         double rho = g[0], rho_old = 1.0, alpha = 1.0, omega = 1.0;
         for (int it = 1; it <= a.maxiter; ++it) {
-            if (rho == 0.0) return 1;
+            // the residual that the previous iteration left is tested with the next
+            // product; when rho underflows to 0 first, here
+            if (rho == 0.0) return it > 1 && passes() ? 0 : 1;
             const double beta = it == 1 ? 0.0 : (rho / rho_old) * (alpha / omega);
 #pragma unroll
             for (int q = 0; q < (NPT ? NPT : cnt); ++q) P[q] = R[q] + beta * (P[q] - omega * V[q]);
@@ -703,11 +712,7 @@ __device__ __forceinline__ void bottom_krylov(Plan& pl, const T* b_in, T* x_out,
             rho_old = rho;
             rho = w[2] - omega * w[3];
         }
-        double u[1] = {0.0};
-#pragma unroll
-        for (int q = 0; q < (NPT ? NPT : cnt); ++q) u[0] = fmax(u[0], unscaled(q));
-        block_reduce<1, 1>(u, red, phase);
-        return u[0] <= stop ? 0 : 2;
+        return passes() ? 0 : 2;
     };
     auto cg = [&](int& iters) -> int {
 #pragma unroll
