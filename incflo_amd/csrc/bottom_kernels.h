@@ -606,12 +606,10 @@ __device__ __forceinline__ void bottom_krylov(Plan& pl, const T* b_in, T* x_out,
         __syncthreads();
         pl.apply(xs, [&](int q, double v) { dst[q] = Plan::kScaled ? v : S[q] * v; });
     };
-    // |r| of an unknown from its scaled residual (S is 0 elsewhere); the
-    // stopping test needs no more than the hardware reciprocal
-    auto unscaled = [&](int q) {
-        const double s = S[q];
-        return s > 0.0 ? nabs(R[q] * __builtin_amdgcn_rcp(s)) : 0.0;
-    };
+    // 1: the residual of an unknown exceeds stop.  Tested on the
+    // scaled one, |S r| > stop S, which needs no division (0 > 0 fails where S is 0)
+    double stop = 0.0;
+    auto over = [&](int q) { return nabs(R[q]) > stop * S[q] ? 1.0 : 0.0; };
 
     pl.setup([&](int q, double dg) {
         const double s = dg > 0.0 ? 1.0 / sqrt(dg) : 0.0;
@@ -644,14 +642,15 @@ __device__ __forceinline__ void bottom_krylov(Plan& pl, const T* b_in, T* x_out,
         }
     }
     block_reduce<1, 1>(rn0, red, phase);
-    const double rnorm0 = rn0[0], stop = a.rtol * rnorm0;
+    const double rnorm0 = rn0[0];
+    stop = a.rtol * rnorm0;
 
     auto passes = [&]() {
         double u[1] = {0.0};
 #pragma unroll
-        for (int q = 0; q < (NPT ? NPT : cnt); ++q) u[0] = fmax(u[0], unscaled(q));
+        for (int q = 0; q < (NPT ? NPT : cnt); ++q) u[0] = fmax(u[0], over(q));
         block_reduce<1, 1>(u, red, phase);
-        return u[0] <= stop;
+        return u[0] == 0.0;
     };
     // 0: converged, 1: broke down, 2: iteration limit; both from zero
     auto bicgstab = [&](int& iters) -> int {
@@ -672,15 +671,15 @@ __device__ __forceinline__ void bottom_krylov(Plan& pl, const T* b_in, T* x_out,
 #pragma unroll
             for (int q = 0; q < (NPT ? NPT : cnt); ++q) P[q] = R[q] + beta * (P[q] - omega * V[q]);
             product(P, V);
-            // (the norm of the residual the previous iteration left)
+            // (and the test of the residual the previous iteration left)
             double u[2] = {0.0, 0.0};
 #pragma unroll
             for (int q = 0; q < (NPT ? NPT : cnt); ++q) {
                 u[0] += B[q] * V[q];
-                u[1] = fmax(u[1], unscaled(q));
+                u[1] = fmax(u[1], over(q));
             }
             block_reduce<2, 2>(u, red, phase);
-            if (it > 1 && u[1] <= stop) return 0;
+            if (it > 1 && u[1] == 0.0) return 0;
             iters = it;
             if (u[0] == 0.0) return 1;
             alpha = rho / u[0];
@@ -697,10 +696,10 @@ __device__ __forceinline__ void bottom_krylov(Plan& pl, const T* b_in, T* x_out,
                 w[1] += W[q] * R[q];
                 w[2] += B[q] * R[q];
                 w[3] += B[q] * W[q];
-                w[4] = fmax(w[4], unscaled(q));
+                w[4] = fmax(w[4], over(q));
             }
             block_reduce<5, 16>(w, red, phase);
-            if (w[4] <= stop) return 0;
+            if (w[4] == 0.0) return 0;
             if (w[0] == 0.0) return 1;
             omega = w[1] / w[0];
 #pragma unroll
@@ -728,10 +727,10 @@ __device__ __forceinline__ void bottom_krylov(Plan& pl, const T* b_in, T* x_out,
             for (int q = 0; q < (NPT ? NPT : cnt); ++q) {
                 u[0] += R[q] * R[q];
                 u[1] += R[q] * W[q];
-                u[2] = fmax(u[2], unscaled(q));
+                u[2] = fmax(u[2], over(q));
             }
             block_reduce<3, 4>(u, red, phase);
-            if (u[0] == 0.0 || (it > 1 && u[2] <= stop)) return 0;
+            if (u[0] == 0.0 || (it > 1 && u[2] == 0.0)) return 0;
             if (it > a.maxiter) return 2;
             iters = it;
             const double beta = it == 1 ? 0.0 : u[0] / g_old;

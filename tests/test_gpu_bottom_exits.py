@@ -52,3 +52,50 @@ def test_rho_underflow_after_convergence(ctx, b, rtol, k):
     info, _ = _solve(ctx, n, beta, np.array(b) / 4096 * 2.0 ** -k, rtol, bottom_solver="bicgstab",
                      bottom_rtol=rtol, maxiter=20)
     assert info.iters == 1
+
+
+def _dense(n, beta):
+    """-L of the solve above as a matrix (unit cells)"""
+    m = int(np.prod(n))
+    A = np.zeros((m, m))
+    at = lambda p: p[0] + n[0] * (p[1] + n[1] * p[2])
+    for k in range(n[2]):
+        for j in range(n[1]):
+            for i in range(n[0]):
+                r = at((i, j, k))
+                for d in range(3):
+                    for s in (0, 1):
+                        q, f = [i, j, k], [k, j, i]
+                        q[d] += 2 * s - 1
+                        f[2 - d] += s
+                        w = beta[d][tuple(f)]
+                        if 0 <= q[d] < n[d]:
+                            A[r, at(q)] -= w
+                            A[r, r] += w
+                        elif d == 0 and s == 0:
+                            A[r, r] += 2 * w
+    return A
+
+
+@pytest.mark.parametrize("seed", range(6))
+@pytest.mark.parametrize("kind", ["cg", "bicgstab"])
+def test_stopping_test_is_exact(ctx, kind, seed):
+    """The residual after the first step, alpha = (b S S b) / (b S A S b) along the
+    scaled right-hand side, is known to round-off (about 100 eps for 60 unknowns);
+    a bottom_rtol 1e-12 above it has to accept that step and one 1e-12 below it
+    has to go on: smoothing sweeps (CG) or the second half of the iteration."""
+    n = (5, 4, 3)
+    print(f"case bottom exit, stopping test, {kind} seed {seed}", flush=True)
+    rng = np.random.default_rng(seed)
+    beta = [0.5 + rng.random([n[2 - a] + (2 - a == d) for a in range(3)]) for d in range(3)]
+    A = _dense(n, beta)
+    b = rng.standard_normal(len(A))
+    s2 = 1.0 / np.diag(A)
+    p = s2 * b
+    step = (b @ p) / (p @ A @ p) * p
+    ratio = np.max(np.abs(b - A @ step)) / np.max(np.abs(b))
+    for side in (1.0 + 1e-12, 1.0 - 1e-12):
+        _, x = _solve(ctx, n, beta, b, 0.999, bottom_solver=kind,
+                      bottom_rtol=ratio * side, bottom_maxiter=1, maxiter=1, verbose=0)
+        same = np.max(np.abs(x + step)) <= 1e-12 * np.max(np.abs(step))
+        assert same == (side > 1.0)
