@@ -137,10 +137,14 @@ __device__ __forceinline__ long gd_ghost(const GdGeom& g, int d, int side, int i
 }
 
 // x / 6, correctly rounded (Markstein: the quotient by the rounded reciprocal,
-// corrected once by its remainder) in 3 operations for a division's 15 or so
-__device__ __forceinline__ double gd_sixth(double x) {
-    const double r = 1.0 / 6.0, q = x * r;
-    return fma(fma(-6.0, q, x), r, q);
+// corrected once by its remainder) in 3 operations for a division's 15 or so.
+// The remainder is exact while the quotient's last bit is a normal number; below
+// 2^-960 the division itself (no wave of ordinary values takes that branch).
+// Of 0, infinities and NaN the product is the quotient, and its remainder NaN.
+__host__ __device__ __forceinline__ double gd_sixth(double x) {
+    const double r = 1.0 / 6.0, q = x * r, m = fabs(x);
+    if (m >= 0x1p-960 && m < __builtin_inf()) return fma(fma(-6.0, q, x), r, q);
+    return m > 0.0 && m < 0x1p-960 ? x / 6.0 : q;
 }
 
 // The point of this thread in a plane of nx x ny points cut into runs of 256
@@ -163,7 +167,6 @@ inline dim3 plane_grid(int nx, int ny, int nz) { return dim3((nx * ny + 255) / 2
 // result a round trip of its own), and the number of components (NC) and the
 // kind of prediction (EX: a.extrap) are template arguments.
 //   128^3 (velocity extrapolation, edge states of 3 and 2 components): 2.90 -> 2.43 ms
-
 
 // 1. PPM traced values for every (d, n), interior cells
 template <bool EX, int NC>
