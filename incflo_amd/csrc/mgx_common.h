@@ -130,7 +130,9 @@ inline double nodal_omega(const NodalGeom& g, double omega) {
 // the unknowns and their condition, and a level of up to 256 cells solves in
 // the time of the six launches that a further level costs.  Mixed projections
 // of a 256 x 16 x 24 channel 6.6 -> 2.4 ms (bottom 64 x 4 x 6 -> 32 x 2 x 3
-// cells), of a 16 x 248 x 216 one 58 -> 4.2 ms.
+// cells), of a 16 x 248 x 216 one 58 -> 4.2 ms.  Not with a body or an overset
+// mask, whose fixed or covered nodes such levels do not resolve: with a block of
+// masked nodes a 128 x 16 x 16 channel went from 36 cycles to no convergence.
 constexpr long kDeepCells = 256;
 inline int nodal_nlevels(const NodalGeom& g, int max_coarsening_level, bool deep = false) {
     int n[3] = {g.n[0], g.n[1], g.n[2]};

@@ -815,6 +815,14 @@ void NodalSolver::set_mask(const unsigned char* m0, hipStream_t s) {
     mask_on = false;
     mask_fixed = false;
     mask_lv.clear();
+    // a fixed region that a level of 2 or 3 cells no longer resolves can make the
+    // cycle diverge (mgx_common.h), so a mask keeps to the levels of 4 and more
+    const int nl = nodal_nlevels(g0, opts.max_coarsening_level, !m0 && deep_levels(opts));
+    if (nl != nlev) {
+        nlev = nl;  // the solves rebuild H32 and H64
+        H16.built = false;
+        logsig_lvl = -1;
+    }
     if (!m0) return;
     mask_lv.resize(nlev);
     NodalGeom gl = g0, gprev = g0;
