@@ -71,6 +71,7 @@ class MacHierarchy {
     std::vector<MacLevel<T>> L;
     DevBuf bottom_work;
     bool built = false;
+    int used = 0;  // levels of the next V-cycle (the last of them is the bottom)
     // level-0 x holds an initial guess (the correction so far): the next cycle
     // smooths from it instead of from zero
     bool x0_guess = false;
@@ -84,7 +85,8 @@ class MacHierarchy {
     MacHierarchy& operator=(const MacHierarchy&) = delete;
     ~MacHierarchy();
     void drop_graphs();
-    void build(const MacGeom& g0, int nlev);
+    // few: the fewest levels a V-cycle will use (0: all)
+    void build(const MacGeom& g0, int nlev, int few = 0);
     // level-0 beta from FP64 face arrays, then coarsen; with Robin sides the
     // boundary planes of each level are then scaled by rscale(l, d, side)
     // (null: not a Robin side)
@@ -102,6 +104,7 @@ class MacHierarchy {
         bool guess0;
         int* bottom_iters;
         long coarse;  // mac_coarse_cells() at capture
+        int used;
         MGOpts o;
         hipGraphExec_t exec;
     };

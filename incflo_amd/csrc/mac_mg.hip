@@ -27,7 +27,7 @@ void MacHierarchy<T>::drop_graphs() {
 }
 
 template <class T>
-void MacHierarchy<T>::build(const MacGeom& g0, int nlev) {
+void MacHierarchy<T>::build(const MacGeom& g0, int nlev, int few) {
     drop_graphs();  // they hold the old levels' addresses
     L.clear();
     L.resize(nlev);
@@ -58,7 +58,8 @@ void MacHierarchy<T>::build(const MacGeom& g0, int nlev) {
         lv.x2 = lv.x2_buf.template as<T>();
         lv.r = lv.r_buf.template as<T>();
     }
-    bottom_work.alloc(bottom_work_doubles(L.back().g.ncell(), 7) * sizeof(double));
+    bottom_work.alloc(bottom_work_doubles(L[(few ? few : nlev) - 1].g.ncell(), 7) * sizeof(double));
+    used = nlev;
     bottom_prepare<MacRows<T>, T>();
     built = true;
 }
@@ -137,7 +138,7 @@ void MacHierarchy<T>::vcycle(const MGOpts& o, hipStream_t s, int* bottom_iters) 
     const CycleGraph* hit = nullptr;
     for (const CycleGraph& c : cache_)
         if (c.x0 == L[0].x && c.b0 == L[0].b && c.guess0 == guess0 && c.bottom_iters == bottom_iters &&
-            c.coarse == coarse && same_cycle_opts(c.o, o))
+            c.coarse == coarse && c.used == used && same_cycle_opts(c.o, o))
             hit = &c;
     if (!hit) {
         if (cache_.size() >= 16) drop_graphs();
@@ -160,7 +161,7 @@ void MacHierarchy<T>::vcycle(const MGOpts& o, hipStream_t s, int* bottom_iters) 
             if (e == hipSuccess && body_ok) e = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
             if (g) (void)hipGraphDestroy(g);
             if (e == hipSuccess && body_ok) {
-                cache_.push_back(CycleGraph{L[0].x, L[0].b, guess0, bottom_iters, coarse, o, exec});
+                cache_.push_back(CycleGraph{L[0].x, L[0].b, guess0, bottom_iters, coarse, used, o, exec});
                 hit = &cache_.back();
             } else {
                 ok = false;
@@ -181,10 +182,10 @@ void MacHierarchy<T>::vcycle(const MGOpts& o, hipStream_t s, int* bottom_iters) 
 
 static_assert(sizeof(MacCoarseArgs<double>) <= 3072, "coarse-cycle kernel arguments");
 
-// the first level of the one-workgroup coarse cycle (nl - 1: none)
+// the first level of the one-workgroup coarse cycle of a V-cycle of nl levels
+// (nl - 1: none)
 template <class T>
-static int mac_coarse_first(const std::vector<MacLevel<T>>& L) {
-    const int nl = (int)L.size();
+static int mac_coarse_first(const std::vector<MacLevel<T>>& L, int nl) {
     const long maxc = mac_coarse_cells();
     int lc = nl - 1;
     while (lc - 1 >= 1 && L[lc - 1].g.ncell() <= maxc && nl - 1 - (lc - 1) <= kMacCoarseMax) --lc;
@@ -192,9 +193,9 @@ static int mac_coarse_first(const std::vector<MacLevel<T>>& L) {
 }
 
 template <class T>
-static MacCoarseArgs<T> mac_coarse_args(std::vector<MacLevel<T>>& L, int lc, const MGOpts& o, int up) {
+static MacCoarseArgs<T> mac_coarse_args(std::vector<MacLevel<T>>& L, int nl, int lc, const MGOpts& o,
+                                        int up) {
     MacCoarseArgs<T> a{};
-    const int nl = (int)L.size();
     a.nlev = nl - 1 - lc;
     a.nu1 = o.nu1;
     a.nu2 = o.nu2;
@@ -214,14 +215,14 @@ static MacCoarseArgs<T> mac_coarse_args(std::vector<MacLevel<T>>& L, int lc, con
 
 template <class T>
 void MacHierarchy<T>::vcycle_body(const MGOpts& o, hipStream_t s, int* bottom_iters) {
-    const int nl = (int)L.size();
+    const int nl = used;
     // levels lc..nl-2 in one workgroup (lc == nl - 1: none)
-    const int lc = mac_coarse_first(L);
+    const int lc = mac_coarse_first(L, nl);
     // down: x (a guess on level 0) -> x2; up: x2 -> x
     for (int l = 0; l < lc; ++l)
         mac_tile_sweeps(mac_tile_args(L[l], L[l + 1]), l == 0 && x0_guess ? MT_X : MT_ZERO, L[l].x, L[l].x2,
                         o.nu1, true, s);
-    if (lc < nl - 1) mac_coarse_cycle_kernel<T><<<1, 1024, 0, s>>>(mac_coarse_args(L, lc, o, 0));
+    if (lc < nl - 1) mac_coarse_cycle_kernel<T><<<1, 1024, 0, s>>>(mac_coarse_args(L, nl, lc, o, 0));
     {
         MacLevel<T>& lb = L[nl - 1];
         BottomArgs ba{};
@@ -235,7 +236,7 @@ void MacHierarchy<T>::vcycle_body(const MGOpts& o, hipStream_t s, int* bottom_it
         bottom_launch<MacRows<T>, T>(rows, lb.g.ncell(), lb.b, lb.x, ba, s);
     }
     x0_guess = false;
-    if (lc < nl - 1) mac_coarse_cycle_kernel<T><<<1, 1024, 0, s>>>(mac_coarse_args(L, lc, o, 1));
+    if (lc < nl - 1) mac_coarse_cycle_kernel<T><<<1, 1024, 0, s>>>(mac_coarse_args(L, nl, lc, o, 1));
     for (int l = lc - 1; l >= 0; --l)
         mac_tile_sweeps(mac_tile_args(L[l], L[l + 1]), MT_PROLONG, L[l].x2, L[l].x, o.nu2, false, s);
 }
@@ -407,14 +408,16 @@ void MacSolver::solve(double* b, double rtol, double atol, int mode, mgx_solve_i
     const std::vector<const double*>* rs = robin_on ? &rob_ptr : nullptr;
     MGX_REQUIRE(!g.has_a || acoef_set, MGX_ERR_STATE, "Helmholtz solve: a coefficient not set");
     const double* A0 = acoef();
+    const int few = mac_nlevels(g, opts.max_coarsening_level, false);
+    LevelChoice choice(nlev, few, n >> 3 * (few - 1));
     if (mixed) {
-        if (!H32.built || (int)H32.L.size() != nlev) { H32.build(g, nlev); h32_beta = h32_a = false; }
+        if (!H32.built || (int)H32.L.size() != nlev) { H32.build(g, nlev, few); h32_beta = h32_a = false; }
         if (!h32_beta) { H32.set_beta(braw0, s, rs); h32_beta = true; }
         if (A0 && !h32_a) { H32.set_acoef(A0, s); h32_a = true; }
         res32.alloc(n * sizeof(float));
         H32.L[0].b = res32.as<float>();
     } else {
-        if (!H64.built || (int)H64.L.size() != nlev) { H64.build(g, nlev); h64_beta = h64_a = false; }
+        if (!H64.built || (int)H64.L.size() != nlev) { H64.build(g, nlev, few); h64_beta = h64_a = false; }
         if (!h64_beta) { H64.set_beta(braw0, s, rs); h64_beta = true; }
         if (A0 && !h64_a) { H64.set_acoef(A0, s); h64_a = true; }
         res64.alloc(n * sizeof(double));
@@ -434,14 +437,17 @@ void MacSolver::solve(double* b, double rtol, double atol, int mode, mgx_solve_i
     const dim3 gr = grid3(g.n[0], g.n[1], g.n[2]);
     unsigned long long* nrm = scal.as<unsigned long long>() + 1;
 
-    zero_u64_kernel<<<1, 64, 0, s>>>(nrm, 1);
-    if (mixed)
-        mac_resid_kernel<double, float, MK_RESID><<<gr, block3(), 0, s>>>(
-            kg, c64, b0[0], b0[1], b0[2], A0, b, phi, nullptr, nullptr, res32.as<float>(), nrm);
-    else
-        mac_resid_kernel<double, double, MK_RESID><<<gr, block3(), 0, s>>>(
-            kg, c64, b0[0], b0[1], b0[2], A0, b, phi, nullptr, nullptr, res64.as<double>(), nrm);
-    const double r0 = read_norm(1, s);
+    auto residual = [&]() {
+        zero_u64_kernel<<<1, 64, 0, s>>>(nrm, 1);
+        if (mixed)
+            mac_resid_kernel<double, float, MK_RESID><<<gr, block3(), 0, s>>>(
+                kg, c64, b0[0], b0[1], b0[2], A0, b, phi, nullptr, nullptr, res32.as<float>(), nrm);
+        else
+            mac_resid_kernel<double, double, MK_RESID><<<gr, block3(), 0, s>>>(
+                kg, c64, b0[0], b0[1], b0[2], A0, b, phi, nullptr, nullptr, res64.as<double>(), nrm);
+        return read_norm(1, s);
+    };
+    const double r0 = residual();
     const double tol = std::max(atol, rtol * bnorm);
     double rn = r0;
     int it = 0;
@@ -454,6 +460,7 @@ void MacSolver::solve(double* b, double rtol, double atol, int mode, mgx_solve_i
         double* pout = (phi == phi_a.as<double>()) ? phi_b.as<double>() : phi_a.as<double>();
         int ran = 1;
         const double prev = rn;
+        H32.used = H64.used = choice.levels();
         if (mixed) {
             // further FP32 cycles on the same FP64 residual, each from the
             // correction so far
@@ -469,9 +476,14 @@ void MacSolver::solve(double* b, double rtol, double atol, int mode, mgx_solve_i
             mac_resid_kernel<double, double, MK_UPDRES><<<gr, block3(), 0, s>>>(
                 kg, c64, b0[0], b0[1], b0[2], A0, b, phi, H64.L[0].x, pout, res64.as<double>(), nrm);
         }
-        phi = pout;
         rn = read_norm(1, s);
         vcycles += ran;
+        if (!choice.step(prev, rn, ran)) {
+            --it;
+            rn = residual();
+            continue;
+        }
+        phi = pout;
         if (opts.verbose)
             fprintf(stderr, "mgx MAC MLMG: iter %d |r| %.6e rel %.3e\n", it, rn,
                     bnorm > 0 ? rn / bnorm : rn);

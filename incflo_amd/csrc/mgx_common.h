@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <cstdio>
 #include <stdexcept>
@@ -148,5 +149,63 @@ inline int nodal_nlevels(const NodalGeom& g, int max_coarsening_level, bool deep
     }
     return nl;
 }
+
+// Which levels a solve's V-cycles use: all of them, or only those of 4 cells and
+// more with the bottom solve on the last such level.  The levels below save most
+// solves the larger bottom, but with anisotropic cells or coefficients that jump
+// by orders of magnitude a cycle through them can contract slowly or diverge
+// where the other does not (MAC, 40 x 24 x 32 cells of 2:1:1: 88 cycles without
+// them, no convergence with them; smooth coefficients on cubes: 9 either way).
+// Each solve starts with all levels and leaves them at the second step in a row
+// that contracts by less than kDeepRho per cycle (kDeepRhoLarge where the other
+// bottom is beyond the register variants and a cycle with it costs several
+// without), or at the first one by less than kBadRho; a step that raises the
+// residual is discarded.  The other choice stays unless it
+// contracts by less than kFewRho per cycle over kWindow cycles, too little to
+// converge in 100 (a Krylov solve of a large bottom that stops at its iteration
+// limit): then the better of the two over such windows.
+constexpr double kDeepRho = 0.3, kDeepRhoLarge = 0.5, kBadRho = 0.8, kFewRho = 0.9;
+constexpr int kWindow = 8;
+struct LevelChoice {
+    int all, few;
+    double leave;
+    bool deep, left = false;     // all levels now; they have been left once
+    bool slow = false;           // the step before was slower than `leave`
+    double rho[2] = {0.0, 0.0};  // contraction per cycle over the last window: few levels, all levels
+    double first = 0.0;          // residual norm before the window's first cycle
+    int n = 0;                   // cycles of the window so far
+    // few_n: unknowns of the bottom of few_levels
+    LevelChoice(int all_levels, int few_levels, long few_n)
+        : all(all_levels), few(few_levels), leave(few_n > 1024 ? kDeepRhoLarge : kDeepRho),
+          deep(all_levels > few_levels) {}
+    int levels() const { return deep ? all : few; }
+    // after a step of `ran` cycles from residual norm prev to rn; false: discard it
+    bool step(double prev, double rn, int ran) {
+        if (all == few) return true;
+        if (!left) {
+            const double c = rn < prev ? std::pow(rn / prev, 1.0 / ran) : 1.0;
+            const bool was = slow;
+            slow = c > leave;
+            if (!slow || (!was && c <= kBadRho)) return true;
+            deep = false;
+            left = true;
+            return rn < prev;
+        }
+        if (n == 0) first = prev;
+        n += ran;
+        if (deep && !(rn < 2.0 * first)) {
+            rho[1] = HUGE_VAL;
+            deep = false;
+            n = 0;
+            return rn < prev;
+        }
+        if (n >= kWindow) {
+            rho[deep] = std::pow(rn / first, 1.0 / n);
+            if (rho[deep] > kFewRho && rho[!deep] < rho[deep]) deep = !deep;
+            n = 0;
+        }
+        return true;
+    }
+};
 
 }  // namespace mgx

@@ -179,7 +179,9 @@ class NodalHierarchy {
     std::vector<MGLevel<T>> L;
     DevBuf bottom_work;
     LaunchTimer* timer = nullptr;  // times the finest-level smoother sweeps
-    void build(const NodalGeom& g0, int nlev);
+    int used = 0;  // levels of the next V-cycle (the last of them is the bottom)
+    // few: the fewest levels a V-cycle will use (0: all)
+    void build(const NodalGeom& g0, int nlev, int few = 0);
     // level-0 sigma (ghosted, same layout) from a double array, then coarsen
     void set_sigma(const double* sig0, hipStream_t s);
     // V-cycle on the correction equation: input L[0].b, output L[0].x.
@@ -221,6 +223,7 @@ class NodalHierarchy {
         bool guess0 = false;
         bool timed = false;
         int* bottom_iters = nullptr;
+        int used = 0;
         MGOpts o;
         hipGraphExec_t exec = nullptr;
         std::vector<T*> xs, x2s;  // buffer roles after the cycle
@@ -241,6 +244,8 @@ class NodalSolver {
     NodalGeom g0;
     MGOpts opts;
     int nlev = 1;
+    // levels of 4 cells and more
+    int few_levels() const { return nodal_nlevels(g0, opts.max_coarsening_level); }
     NodalHierarchy<double> H64;
     NodalHierarchy<float> H32;
     DevBuf sig0_buf;         // level-0 sigma (ghosted, FP64)

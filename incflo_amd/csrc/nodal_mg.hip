@@ -400,7 +400,7 @@ void NodalHierarchy<T>::drop_graphs() {
 }
 
 template <class T>
-void NodalHierarchy<T>::build(const NodalGeom& g0, int nlev) {
+void NodalHierarchy<T>::build(const NodalGeom& g0, int nlev, int few) {
     drop_graphs();
     static bool attr_set = false;
     if (!attr_set) {
@@ -433,7 +433,8 @@ void NodalHierarchy<T>::build(const NodalGeom& g0, int nlev) {
         lv.x2 = lv.x2_buf.template as<T>();
         lv.r = lv.r_buf.template as<T>();
     }
-    bottom_work.alloc(bottom_work_doubles(L.back().g.nnode(), 27) * sizeof(double));
+    bottom_work.alloc(bottom_work_doubles(L[(few ? few : nlev) - 1].g.nnode(), 27) * sizeof(double));
+    used = nlev;
     built = true;
 }
 
@@ -534,7 +535,7 @@ void NodalHierarchy<T>::vcycle(const MGOpts& o, hipStream_t s, int* bottom_iters
     CycleGraph* hit = nullptr;
     for (auto& c : cache_)
         if (c.x0 == L[0].x && c.b0 == L[0].b && c.ready0 == ready0 && c.guess0 == guess0 &&
-            c.timed == timed &&
+            c.timed == timed && c.used == used &&
             c.bottom_iters == bottom_iters && same_opts(c.o, o))
             hit = &c;
     if (!hit) {
@@ -545,6 +546,7 @@ void NodalHierarchy<T>::vcycle(const MGOpts& o, hipStream_t s, int* bottom_iters
         c.guess0 = guess0;
         c.timed = timed;
         c.bottom_iters = bottom_iters;
+        c.used = used;
         c.o = o;
         const bool saved_ready = x0_ready;
         const bool saved_guess = x0_guess;
@@ -609,7 +611,7 @@ void NodalHierarchy<T>::vcycle(const MGOpts& o, hipStream_t s, int* bottom_iters
 
 template <class T>
 void NodalHierarchy<T>::vcycle_body(const MGOpts& o, hipStream_t s, int* bottom_iters) {
-    const int nl = (int)L.size();
+    const int nl = used;
     // levels lc..nl-1 run in the LDS-resident coarse kernel (tuning table
     // coarse_nodes, when they fit); lc == nl - 1: the bottom solve alone
     constexpr size_t kLdsBudget = 150 * 1024;
@@ -777,7 +779,7 @@ static void remove_mean(NodalSolver& S, double* a, long n, hipStream_t s) {
 }
 
 void NodalSolver::prepare_h32(hipStream_t s) {
-    if (!H32.built || (int)H32.L.size() != nlev) { H32.build(g0, nlev); h32_sigma = false; }
+    if (!H32.built || (int)H32.L.size() != nlev) { H32.build(g0, nlev, few_levels()); h32_sigma = false; }
     if (!h32_sigma) { H32.set_sigma(sigma0(), s); h32_sigma = true; }
     res32.alloc(g0.nnode() * sizeof(float));
     H32.L[0].b = res32.as<float>();
@@ -865,7 +867,7 @@ void NodalSolver::prepare_h16(hipStream_t s) {
         T.x = T.xa.as<__half>();
         T.x2 = T.xb.as<__half>();
         const NodalGeom gs = coarsen(T.g);
-        T.sub.build(gs, nlev - 1);
+        T.sub.build(gs, nlev - 1, std::max(1, few_levels() - 1));
         T.sub.timer = nullptr;
         T.sub_b.alloc(gs.nnode() * sizeof(float));
         T.sub.L[0].b = T.sub_b.as<float>();
@@ -945,7 +947,7 @@ void NodalSolver::vcycle16(hipStream_t s) {
 }
 
 static void prepare_h64(NodalSolver& S, hipStream_t s) {
-    if (!S.H64.built || (int)S.H64.L.size() != S.nlev) S.H64.build(S.g0, S.nlev);
+    if (!S.H64.built || (int)S.H64.L.size() != S.nlev) S.H64.build(S.g0, S.nlev, S.few_levels());
     // level-0 sigma of the FP64 hierarchy is the solver's own array
     if (S.H64.L[0].sig != S.sigma0()) {
         S.H64.L[0].sig_buf.release();
@@ -1545,6 +1547,8 @@ void NodalSolver::solve(double* b, double rtol, double atol, int mode, mgx_solve
     int prec = vprec;
     int stall = 0;
     int ncyc = opts.cycles_per_update;  // FP32 cycles of the next refinement step
+    const int few = few_levels();
+    LevelChoice choice(nlev, few, g0.nnode() >> 3 * (few - 1));
     while (!conv && it < opts.maxiter && std::isfinite(rn)) {
         ++it;
         double* pout = other();
@@ -1555,6 +1559,8 @@ void NodalSolver::solve(double* b, double rtol, double atol, int mode, mgx_solve
             ++lsteps;
             learned_guess(rn);
         }
+        H32.used = H64.used = choice.levels();
+        if (half) H16.sub.used = std::max(1, choice.levels() - 1);
         if (prec == P16) vcycle16(s);
         else if (prec == P32) {
             // further FP32 cycles on the same FP64 residual, each from the
@@ -1568,6 +1574,11 @@ void NodalSolver::solve(double* b, double rtol, double atol, int mode, mgx_solve
         vcycles += ran;
         const double prev = rn;
         rn = update(prec, pout, rn);
+        if (!choice.step(prev, rn, ran)) {
+            --it;
+            rn = residual(prec, prev);
+            continue;
+        }
         phi = pout;
         if (prec == P32 && opts.cycles_per_update > 1 && rn > tol && rn < prev) {
             // the next step runs the cycles the measured per-cycle contraction
@@ -1593,6 +1604,9 @@ void NodalSolver::solve(double* b, double rtol, double atol, int mode, mgx_solve
             }
         }
     }
+    H32.used = (int)H32.L.size();
+    H64.used = (int)H64.L.size();
+    if (half) H16.sub.used = (int)H16.sub.L.size();
     if (sing) remove_mean(*this, phi, nn, s);
     int bot = 0;
     MGX_HIP(hipMemcpyAsync(&bot, ibuf.p, sizeof(int), hipMemcpyDeviceToHost, s));
