@@ -277,11 +277,10 @@ MGX_API int mgx_mac_set_options(mgx_mac h, const mgx_mlmg_opts* o) {
     return guarded(h->ctx, [&] {
         MGOpts m;
         to_opts(o, m);
-        const bool relevel = m.max_coarsening_level != h->opts.max_coarsening_level ||
-                             deep_levels(m) != deep_levels(h->opts);
+        const bool relevel = m.max_coarsening_level != h->opts.max_coarsening_level;
         h->opts = m;
         if (relevel) h->dirty = true;
-        else h->solver.opts = h->opts;
+        else if (!h->dirty) h->solver.set_options(m);
     });
 }
 
@@ -651,7 +650,8 @@ MGX_API int mgx_mac_set_eb_cylinder(mgx_mac h, double cx, double cy, double r) {
         h->eb_cyl[1] = cy;
         h->eb_cyl[2] = r;
         // cut cells on a grid two or three cells wide do not represent the body
-        h->solver.set_deep(false);
+        h->solver.deep = false;
+        if (!h->dirty) h->solver.set_options(h->opts);
         if (!h->dirty) h->build_eb();
     });
 }

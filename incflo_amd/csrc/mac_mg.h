@@ -119,7 +119,8 @@ class MacSolver {
     MGOpts opts;
     int nlev = 1;
     bool deep = true;     // levels down to 2 cells where the bottom would be large (nodal_nlevels)
-    void set_deep(bool on);
+    // options with the same max_coarsening_level, on the set-up as it is
+    void set_options(const MGOpts& o);
     MacHierarchy<double> H64;
     MacHierarchy<float> H32;
     DevBuf beta0[3];      // level-0 face coefficients (FP64)

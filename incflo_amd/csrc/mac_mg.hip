@@ -284,8 +284,9 @@ void MacSolver::setup(const MacGeom& g, const MGOpts& o) {
     beta0s_ok = false;
 }
 
-void MacSolver::set_deep(bool on) {
-    deep = on;
+// (the solves rebuild H32 and H64 for a new level count)
+void MacSolver::set_options(const MGOpts& o) {
+    opts = o;
     nlev = mac_nlevels(g0, opts.max_coarsening_level, deep && deep_levels(opts));
 }
 

@@ -328,11 +328,10 @@ MGX_API int mgx_nodal_set_options(mgx_nodal h, const mgx_mlmg_opts* o) {
         MGX_REQUIRE(o != nullptr, MGX_ERR_ARG, "null options");
         MGOpts m;
         to_opts(o, m);
-        const bool relevel = m.max_coarsening_level != h->opts.max_coarsening_level ||
-                             deep_levels(m) != deep_levels(h->opts);
+        const bool relevel = m.max_coarsening_level != h->opts.max_coarsening_level;
         h->opts = m;
         if (relevel) h->dirty = true;
-        else h->solver.opts = m;
+        else if (!h->dirty) h->solver.set_options(m);
     });
 }
 

@@ -272,6 +272,9 @@ class NodalSolver {
 
     ~NodalSolver();
     void setup(const NodalGeom& g, const MGOpts& o);
+    // options with the same max_coarsening_level, on the set-up as it is
+    void set_options(const MGOpts& o);
+    void relevel(bool deep);
     double* sigma0() { return sig0_buf.as<double>(); }
     // Mixed-mode V-cycle with an FP16-stored finest level (FP32 arithmetic):
     // the operator is scaled to L' = L dx0^2 / sigma_max and the residual to

@@ -808,6 +808,20 @@ static __global__ void mask_zero_kernel(const unsigned char* __restrict__ m, dou
     if (id < n && !m[id]) b[id] = 0.0;
 }
 
+// the level count of the options; the solves rebuild H32 and H64 for a new one
+void NodalSolver::relevel(bool deep) {
+    const int nl = nodal_nlevels(g0, opts.max_coarsening_level, deep && deep_levels(opts));
+    if (nl == nlev) return;
+    nlev = nl;
+    H16.built = false;
+    logsig_lvl = -1;
+}
+
+void NodalSolver::set_options(const MGOpts& o) {
+    opts = o;
+    relevel(!mask_on);
+}
+
 void NodalSolver::set_mask(const unsigned char* m0, hipStream_t s) {
     // captured V-cycles hold the old mask pointers
     H64.drop_graphs();
@@ -819,12 +833,7 @@ void NodalSolver::set_mask(const unsigned char* m0, hipStream_t s) {
     mask_lv.clear();
     // a fixed region that a level of 2 or 3 cells no longer resolves can make the
     // cycle diverge (mgx_common.h), so a mask keeps to the levels of 4 and more
-    const int nl = nodal_nlevels(g0, opts.max_coarsening_level, !m0 && deep_levels(opts));
-    if (nl != nlev) {
-        nlev = nl;  // the solves rebuild H32 and H64
-        H16.built = false;
-        logsig_lvl = -1;
-    }
+    relevel(!m0);
     if (!m0) return;
     mask_lv.resize(nlev);
     NodalGeom gl = g0, gprev = g0;
