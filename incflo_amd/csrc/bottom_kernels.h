@@ -6,12 +6,16 @@
 // unknowns, so the time is a serial chain of stencil products, reductions and
 // barriers; no other CU can help without device-wide barriers, which cost as
 // much as the whole product.  Hence
-//   * the rows are assembled once per solve (27 or 7 coefficients, scaled
-//     symmetrically by the diagonal: S L S with S = |diag|^-1/2, which evens out
-//     wall rows and small cut cells and needs fewer iterations), and stay in
-//     registers up to 1024 unknowns; larger levels stream them from L2;
+//   * the operator is scaled symmetrically by the diagonal (S L S with S =
+//     |diag|^-1/2), which evens out wall rows and small cut cells and needs fewer
+//     iterations.  Its rows (27 or 7 coefficients) are assembled once per solve:
+//     in registers up to 512 unknowns (1024 of 27, 2048 of 7 points for the EB and
+//     cell-centred operators), streamed from L2 above.  On nodal levels of more
+//     than 512 nodes columns of nodes work from the cell coefficients instead,
+//     but for levels up to 4096 nodes that 512 threads do not hold in columns;
 //   * each thread owns fixed unknowns, whose vector elements stay in registers
-//     up to 4096 unknowns; only the multiplied vector goes through LDS;
+//     up to 4096 unknowns; only the multiplied vector goes through LDS, up to
+//     19200 unknowns;
 //   * reductions run on DPP row shifts and one barrier, several values at a
 //     time: BiCGStab takes two reductions per iteration (the next rho by its
 //     recurrence, the residual norm together with the next product), CG one
@@ -20,7 +24,7 @@
 // with its vectors and index divisions in LDS or global memory before it:
 //   nodal 1280 nodes (120 x 72 x 56 channel)          592 -> 150 us
 //   nodal 2275 nodes (256 x 16 x 24 channel)         2370 -> 527 us
-//   nodal 10440 nodes (224 x 232 x 88 channel)       6730 -> 3920 us
+//   nodal 10440 nodes (224 x 232 x 88 channel)       6730 -> 3680 us
 //   EB nodal 425 nodes (256 x 64 x 64 channel)       1130 -> 70 us
 //   MAC 480 cells (160 x 24 x 16 channel at 2 levels) 1320 -> 200 us
 #pragma once
@@ -41,7 +45,7 @@ namespace mgx {
 constexpr int kBottomSmooths = 8;
 
 struct BottomArgs {
-    double* work;    // coefficients and, on large levels, vectors: (NS + 7) n doubles
+    double* work;    // BottomPlan::work doubles
     int kind;        // MGX_BOTTOM_*
     int maxiter;
     double rtol;
@@ -128,12 +132,12 @@ __device__ __forceinline__ void block_reduce(double (&v)[NV], BottomRed& red, in
 template <class TS>
 struct NodalRows {
     static constexpr int NS = 27;
-    static constexpr bool kRedBlack = false;
+    static constexpr bool kRedBlack = false, kNodal = true;
     KGeom g;
     Coef<double> c;
     const TS* sig;
     const unsigned char* m;  // overset mask, may be null
-    __device__ int dim(int d) const { return g.nn[d]; }
+    __host__ __device__ int dim(int d) const { return g.nn[d]; }
     __device__ int per(int d) const { return g.per[d]; }
     __device__ bool row(int id, int i, int j, int k, double (&C)[NS]) const {
         double S[2][2][2];
@@ -172,14 +176,18 @@ struct NodalRows {
 };
 
 // ---- the scaled operator A = -S L S, S = |diag|^-1/2, over the workgroup ----
-// A plan maps unknowns to threads (id(q), live(q), q < NPT or count()) and
-// multiplies.  setup() returns the diagonal per unknown (0: not an unknown),
-// scale() receives S through xs, apply() reads the vector in xs.
+// A plan maps unknowns to threads (q < NPT or count(); each(f) calls f(q, id) for
+// those that are unknowns of the level) and multiplies.  setup() returns the
+// diagonal per unknown (0: not an unknown), scale() receives S through xs,
+// apply() reads the vector in xs.  kDirect: the vectors of all threads together
+// are laid out by id, so that apply() reads them where they are.
 
 // Coefficient rows: in registers (CREG), or slot-major in global memory.  NPT
-// 0: any number of unknowns, nothing per unknown in registers.
-template <class Rows, int NPT_, bool CREG>
+// 0: any number of unknowns, nothing per unknown in registers; DIRECT: their
+// multiplied vector is not copied (it would not fit LDS).
+template <class Rows, int NPT_, bool CREG, bool DIRECT = false>
 struct RowPlan {
+    static constexpr bool kDirect = DIRECT;
     static constexpr int NPT = NPT_, NS = Rows::NS;
     static constexpr bool kRedBlack = Rows::kRedBlack;
     static constexpr bool kScaled = true;  // apply() multiplies by A, not -L
@@ -200,6 +208,12 @@ struct RowPlan {
     __device__ int count() const { return (n - tid + nt - 1) / nt; }
     __device__ int id(int q) const { return tid + q * nt; }
     __device__ bool live(int q) const { return NPT == 0 || id(q) < n; }
+    template <class F>
+    __device__ void each(F f) const {
+#pragma unroll
+        for (int q = 0; q < (NPT ? NPT : count()); ++q)
+            if (live(q)) f(q, id(q));
+    }
     __device__ void point(int id, int& i, int& j, int& k) const {
         i = id % d0;
         const int t = id / d0;
@@ -345,7 +359,7 @@ __device__ __forceinline__ double col_node(const double (&x0)[3][3], const doubl
 template <class TS, int NPT_>
 struct ColPlan {
     static constexpr int NPT = NPT_;
-    static constexpr bool kRedBlack = false, kScaled = false;
+    static constexpr bool kRedBlack = false, kScaled = false, kDirect = false;
     const NodalRows<TS>& op;
     int na, nbk, nm, nseg;      // nodes along the two cross axes and the march axis
     int sa, sb, sm;             // id strides
@@ -413,6 +427,12 @@ struct ColPlan {
     __device__ bool live(int q) const { return on && m0 + q < nm; }
     __device__ int id(int q) const { return sa * ca + sb * cb + sm * min(m0 + q, nm - 1); }
     template <class F>
+    __device__ void each(F f) const {
+#pragma unroll
+        for (int q = 0; q < NPT; ++q)
+            if (live(q)) f(q, id(q));
+    }
+    template <class F>
     __device__ void setup(F put) {
 #pragma unroll
         for (int q = 0; q < NPT; ++q) {
@@ -462,17 +482,17 @@ struct ColPlan {
 };
 
 // The same for levels whose vectors do not fit the registers: a thread owns
-// whole columns along the shortest axis (at least 256 columns from 4096 nodes
-// on), its vectors lie in global memory in the order it visits them.
+// segments of `len` nodes of columns along `axis` (items, column fastest), its
+// vectors lie in global memory in the order it visits them.
 template <class TS>
 struct WidePlan {
     static constexpr int NPT = 0;
-    static constexpr bool kRedBlack = false, kScaled = false;
+    static constexpr bool kRedBlack = false, kScaled = false, kDirect = false;
     const NodalRows<TS>& op;
-    int axis, a, b, na, ncol, nm, sa, sb, sm;
+    int axis, len, a, b, na, ncol, nm, sa, sb, sm, items;
     Coef<double> c;
-    __device__ WidePlan(const NodalRows<TS>& o, int axis_)
-        : op(o), axis(axis_), a(axis_ == 0 ? 1 : 0), b(axis_ == 2 ? 1 : 2), c(o.c) {
+    __device__ WidePlan(const NodalRows<TS>& o, int axis_, int len_)
+        : op(o), axis(axis_), len(len_), a(axis_ == 0 ? 1 : 0), b(axis_ == 2 ? 1 : 2), c(o.c) {
         const int st[3] = {1, o.dim(0), o.dim(0) * o.dim(1)};
         na = o.dim(a);
         ncol = na * o.dim(b);
@@ -480,6 +500,7 @@ struct WidePlan {
         sa = st[a];
         sb = st[b];
         sm = st[axis];
+        items = ncol * ((nm + len - 1) / len);
         c.edge[0] = o.c.edge[a];
         c.edge[1] = o.c.edge[b];
         c.edge[2] = o.c.edge[axis];
@@ -488,14 +509,27 @@ struct WidePlan {
         c.face[2] = o.c.face[axis];
     }
     __device__ int size() const { return ncol * nm; }
-    __device__ int cols() const { return (ncol - (int)threadIdx.x + (int)blockDim.x - 1) / (int)blockDim.x; }
-    __device__ int count() const { return (int)threadIdx.x < ncol ? cols() * nm : 0; }
+    // this thread's items
+    __device__ int mine() const {
+        return (int)threadIdx.x < items ? (items - (int)threadIdx.x + (int)blockDim.x - 1) / (int)blockDim.x : 0;
+    }
+    __device__ int count() const { return mine() * len; }
     // doubles a vector takes (every thread's share padded to the longest)
-    __device__ long stride() const { return (long)((ncol + blockDim.x - 1) / blockDim.x) * nm * blockDim.x; }
-    __device__ bool live(int) const { return true; }
-    __device__ int id(int q) const {
-        const int w = q / nm, cc = threadIdx.x + w * blockDim.x;
-        return sa * (cc % na) + sb * (cc / na) + sm * (q - w * nm);
+    __device__ long stride() const { return (long)((items + blockDim.x - 1) / blockDim.x) * len * blockDim.x; }
+    // f(w, ca, cb, m0, m1): item w, its column and its nodes m0 .. m1 - 1
+    template <class F>
+    __device__ void each_item(F f) const {
+        const int cnt = mine();
+        for (int w = 0; w < cnt; ++w) {
+            const int it = threadIdx.x + w * blockDim.x, sg = it / ncol, cc = it - sg * ncol, cb = cc / na;
+            f(w, cc - cb * na, cb, sg * len, min(sg * len + len, nm));
+        }
+    }
+    template <class F>
+    __device__ void each(F f) const {
+        each_item([&](int w, int ca, int cb, int m0, int m1) {
+            for (int m = m0; m < m1; ++m) f(w * len + m - m0, sa * ca + sb * cb + sm * m);
+        });
     }
     __device__ void cells(double (&s)[2][2], int ca, int cb, int l) const {
         const int g3[3] = {1, op.g.sg[0], op.g.sg[0] * op.g.sg[1]};
@@ -505,11 +539,10 @@ struct WidePlan {
     }
     template <class F>
     __device__ void setup(F put) {
-        for (int w = 0; w < (count() ? cols() : 0); ++w) {
-            const int cc = threadIdx.x + w * blockDim.x, ca = cc % na, cb = cc / na;
+        each_item([&](int w, int ca, int cb, int m0, int m1) {
             double s0[2][2], s1[2][2];
-            cells(s0, ca, cb, 0);
-            for (int m = 0; m < nm; ++m) {
+            cells(s0, ca, cb, m0);
+            for (int m = m0; m < m1; ++m) {
                 cells(s1, ca, cb, m + 1);
                 double t = 0.0;
 #pragma unroll
@@ -519,15 +552,15 @@ struct WidePlan {
                 }
                 const int e = sa * ca + sb * cb + sm * m, i = e % op.dim(0), v = e / op.dim(0);
                 const bool free = t > 0.0 && !node_fixed(op.g, op.m, e, i, v % op.dim(1), v / op.dim(1));
-                put(w * nm + m, free ? c.diag4 * t : 0.0);
+                put(w * len + m - m0, free ? c.diag4 * t : 0.0);
             }
-        }
+            for (int m = m1; m < m0 + len; ++m) put(w * len + m - m0, 0.0);
+        });
     }
     __device__ void scale(const double*) {}
     template <class F>
     __device__ void apply(const double* xs, F put) {
-        for (int w = 0; w < (count() ? cols() : 0); ++w) {
-            const int cc = threadIdx.x + w * blockDim.x, ca = cc % na, cb = cc / na;
+        each_item([&](int w, int ca, int cb, int m0, int m1) {
             int o[3][3];
 #pragma unroll
             for (int r = 0; r < 3; ++r)
@@ -542,13 +575,13 @@ struct WidePlan {
 #pragma unroll
                     for (int q = 0; q < 3; ++q) x[r][q] = xs[o[r][q] + e];
             };
-            plane(X[0], -1);
-            plane(X[1], 0);
-            cells(G[0], ca, cb, 0);
-            for (int m = 0; m < nm; ++m) {
+            plane(X[0], m0 - 1);
+            plane(X[1], m0);
+            cells(G[0], ca, cb, m0);
+            for (int m = m0; m < m1; ++m) {
                 plane(X[2], m + 1);
                 cells(G[1], ca, cb, m + 1);
-                put(w * nm + m, -col_node(X[0], X[1], X[2], G[0], G[1], c));
+                put(w * len + m - m0, -col_node(X[0], X[1], X[2], G[0], G[1], c));
 #pragma unroll
                 for (int r = 0; r < 3; ++r)
 #pragma unroll
@@ -559,7 +592,8 @@ struct WidePlan {
 #pragma unroll
                 for (int q = 0; q < 4; ++q) G[0][q >> 1][q & 1] = G[1][q >> 1][q & 1];
             }
-        }
+            for (int m = m1; m < m0 + len; ++m) put(w * len + m - m0, 0.0);
+        });
     }
 };
 
@@ -579,8 +613,8 @@ struct OwnVec<0> {
     __device__ double& operator[](int q) { return p[(long)q * nt]; }
 };
 
-// xs: size() doubles (LDS or global memory) for the multiplied vector; vw: 7
-// stride() doubles for the vectors (NPT 0 only)
+// xs: size() doubles (LDS or global memory) for the multiplied vector (not
+// kDirect); vw: 7 stride() doubles for the vectors (NPT 0 only)
 template <class Plan, class T>
 __device__ __forceinline__ void bottom_krylov(Plan& pl, const T* b_in, T* x_out, const BottomArgs& a,
                                               double* xs, double* vw, BottomRed& red) {
@@ -600,11 +634,11 @@ __device__ __forceinline__ void bottom_krylov(Plan& pl, const T* b_in, T* x_out,
     // dst = A src; src through xs.  The next write of xs comes after a
     // reduction or barrier that every read precedes.
     auto product = [&](OwnVec<NPT>& src, OwnVec<NPT>& dst) {
-#pragma unroll
-        for (int q = 0; q < (NPT ? NPT : cnt); ++q)
-            if (pl.live(q)) xs[pl.id(q)] = Plan::kScaled ? src[q] : S[q] * src[q];
+        const double* x = xs;
+        if constexpr (Plan::kDirect) x = src.p - tid;
+        else pl.each([&](int q, int id) { xs[id] = Plan::kScaled ? src[q] : S[q] * src[q]; });
         __syncthreads();
-        pl.apply(xs, [&](int q, double v) { dst[q] = Plan::kScaled ? v : S[q] * v; });
+        pl.apply(x, [&](int q, double v) { dst[q] = Plan::kScaled ? v : S[q] * v; });
     };
     // 1: the residual of an unknown exceeds stop.  Tested on the
     // scaled one, |S r| > stop S, which needs no division (0 > 0 fails where S is 0)
@@ -612,22 +646,24 @@ __device__ __forceinline__ void bottom_krylov(Plan& pl, const T* b_in, T* x_out,
     auto over = [&](int q) { return nabs(R[q]) > stop * S[q] ? 1.0 : 0.0; };
 
     pl.setup([&](int q, double dg) {
-        const double s = dg > 0.0 ? 1.0 / sqrt(dg) : 0.0;
-        S[q] = s;
-        if (pl.live(q)) xs[pl.id(q)] = s;
-    });
-    __syncthreads();
-    pl.scale(xs);
-    double st0[2] = {0.0, 0.0};
-#pragma unroll
-    for (int q = 0; q < (NPT ? NPT : cnt); ++q) {
+        S[q] = dg > 0.0 ? 1.0 / sqrt(dg) : 0.0;
         B[q] = 0.0;
+    });
+    if constexpr (Plan::kScaled) {
+        const double* x = xs;
+        if constexpr (Plan::kDirect) x = S.p - tid;
+        else pl.each([&](int q, int id) { xs[id] = S[q]; });
+        __syncthreads();
+        pl.scale(x);
+    }
+    double st0[2] = {0.0, 0.0};
+    pl.each([&](int q, int id) {
         if (S[q] > 0.0) {
-            B[q] = (double)b_in[pl.id(q)];
+            B[q] = (double)b_in[id];
             st0[0] += B[q];
             st0[1] += 1.0;
         }
-    }
+    });
     block_reduce<2, 0>(st0, red, phase);
     const double nfree = st0[1];
     const double bmean = (a.singular && nfree > 0.0) ? st0[0] / nfree : 0.0;
@@ -769,17 +805,16 @@ __device__ __forceinline__ void bottom_krylov(Plan& pl, const T* b_in, T* x_out,
             for (int color = 0; color < (Plan::kRedBlack ? 2 : 1); ++color) {
                 __syncthreads();
                 product(Y, W);
-#pragma unroll
-                for (int q = 0; q < (NPT ? NPT : cnt); ++q) {
-                    if (!pl.live(q)) continue;
+                if constexpr (Plan::kDirect) __syncthreads();  // every read of Y before its update
+                pl.each([&](int q, int id) {
                     if constexpr (Plan::kRedBlack) {
                         int i, j, k;
-                        pl.point(pl.id(q), i, j, k);
+                        pl.point(id, i, j, k);
                         if (((i + j + k) & 1) == color) Y[q] += B[q] - W[q];
                     } else {
                         Y[q] += a.omega * (B[q] - W[q]);
                     }
-                }
+                });
             }
         if (a.kind == MGX_BOTTOM_SMOOTHER) it = smooths;
     }
@@ -792,9 +827,7 @@ __device__ __forceinline__ void bottom_krylov(Plan& pl, const T* b_in, T* x_out,
     __syncthreads();
     block_reduce<1, 0>(xsum, red, phase);
     const double xmean = (a.singular && nfree > 0.0) ? xsum[0] / nfree : 0.0;
-#pragma unroll
-    for (int q = 0; q < (NPT ? NPT : cnt); ++q)
-        if (pl.live(q)) x_out[pl.id(q)] = S[q] > 0.0 ? (T)(Y[q] - xmean) : (T)0;
+    pl.each([&](int q, int id) { x_out[id] = S[q] > 0.0 ? (T)(Y[q] - xmean) : (T)0; });
     if (tid == 0 && a.iters_acc) atomicAdd(a.iters_acc, it);
 }
 
@@ -804,11 +837,8 @@ static __global__ void __launch_bounds__(NT) bottom_kernel(Rows op, const T* b_i
                                                            BottomArgs a) {
     extern __shared__ __align__(16) double bottom_xs[];
     __shared__ BottomRed red;
-    RowPlan<Rows, NPT, CREG> plan(op, a.work);
-    double* vw = a.work + (long)Rows::NS * plan.size();
-    double* xs = bottom_xs;
-    if constexpr (!XLDS) xs = vw + 7L * plan.size();
-    bottom_krylov(plan, b_in, x_out, a, xs, vw, red);
+    RowPlan<Rows, NPT, CREG, !XLDS> plan(op, a.work);
+    bottom_krylov(plan, b_in, x_out, a, bottom_xs, a.work + (long)Rows::NS * plan.size(), red);
 }
 
 // nodal levels of more than 512 nodes: 512 threads, columns along `axis`
@@ -821,115 +851,154 @@ static __global__ void __launch_bounds__(512) bottom_cols_kernel(NodalRows<TS> o
     bottom_krylov(plan, b_in, x_out, a, bottom_xs, nullptr, red);
 }
 
-// nodal levels of more than 4096 nodes (work: 7 strides of at most n + 1024
-// shortest <= 5 n doubles, from 256 columns on)
-template <class TS, class T>
-static __global__ void __launch_bounds__(1024) bottom_wide_kernel(NodalRows<TS> op, int axis, const T* b_in,
-                                                                  T* x_out, BottomArgs a) {
+// nodal levels that those do not hold; XLDS: the multiplied vector fits LDS
+// (compile-time, for LDS instructions instead of generic ones: 20% of the time)
+template <class TS, class T, bool XLDS>
+static __global__ void __launch_bounds__(1024) bottom_wide_kernel(NodalRows<TS> op, int axis, int len,
+                                                                  const T* b_in, T* x_out, BottomArgs a) {
     extern __shared__ __align__(16) double bottom_xs[];
     __shared__ BottomRed red;
-    WidePlan<TS> plan(op, axis);
-    bottom_krylov(plan, b_in, x_out, a, bottom_xs, a.work, red);
+    WidePlan<TS> plan(op, axis, len);
+    double* xs = bottom_xs;
+    if constexpr (!XLDS) xs = a.work + 7 * plan.stride();
+    bottom_krylov(plan, b_in, x_out, a, xs, a.work, red);
 }
 
 constexpr size_t kBottomLds = 150 * 1024;
 
-// doubles of BottomArgs::work for n unknowns of NS-point rows
-inline size_t bottom_work_doubles(long n, int ns) { return (size_t)(ns + 8) * n; }
+// The variant of a level and what it needs, by the number of unknowns and from
+// what a CU's register file holds (512 threads get 256 VGPRs each, 1024 threads
+// 128): vectors 14 VGPRs, 27-point rows 54 and 7-point rows 14 VGPRs per unknown.
+// Rows read from global memory took the 1280-node nodal solve 740 us, columns
+// 150; with spilled rows 8 nodes per column thread took 1900 us at 2275 nodes,
+// without 527.
+struct BottomPlan {
+    enum Kind { REG1, REG2, REG4, COLS4, COLS8, WIDE, ROWS2, ROWS4, ROWS } kind;
+    long n = 0;
+    int axis = 2, len = 0;   // COLS and WIDE
+    unsigned threads = 1024;
+    size_t lds = 0;          // bytes; 0 for WIDE and ROWS: the multiplied vector in global memory
+    size_t work = 0;         // doubles of BottomArgs::work
+};
+
+template <class Rows>
+inline BottomPlan bottom_plan(const Rows& op) {
+    const auto up64 = [](long v) { return (unsigned)((v + 63) / 64 * 64); };
+    const long d[3] = {op.dim(0), op.dim(1), op.dim(2)}, n = d[0] * d[1] * d[2];
+    BottomPlan p;
+    p.n = n;
+    p.lds = (size_t)n * sizeof(double);
+    const auto pick = [&](BottomPlan::Kind kind, int per, size_t work) {
+        p.kind = kind;
+        if (per) p.threads = up64((n + per - 1) / per);
+        p.work = work;
+        return p;
+    };
+    if (n <= 512) return pick(BottomPlan::REG1, 1, 0);
+    if constexpr (Rows::kNodal) {
+        // columns of 4 or 8 nodes in registers, when 512 threads hold the level
+        // along some axis (the first that does)
+        const size_t lds = p.lds + (size_t)op.g.sg[0] * op.g.sg[1] * op.g.sg[2] * sizeof(*op.sig);
+        for (int npt : {4, 8})
+            for (int axis = 2; axis >= 0 && lds <= kBottomLds; --axis) {
+                const long threads = n / d[axis] * ((d[axis] + npt - 1) / npt);
+                if (threads > 512) continue;
+                p.axis = axis;
+                p.lds = lds;
+                p.threads = up64(threads);
+                return pick(npt == 4 ? BottomPlan::COLS4 : BottomPlan::COLS8, 0, 0);
+            }
+        // (13 x 26 x 10 nodes, 20 BiCGStab iterations: 1.41 ms, segments 1.54)
+        if (n <= 4096) return pick(BottomPlan::ROWS4, 4, (size_t)Rows::NS * n);
+        // segments of columns along y or z (x: the threads of a wave would not read
+        // neighbouring nodes, up to 2.6 times slower) for 1024 threads: fewest
+        // planes in all, twice, and on the busiest thread, with two more planes
+        // per segment than nodes.  20 BiCGStab iterations, whole columns / halves
+        // / thirds: 46^3 nodes 42.9 / 39.3 / 40.2 ms, 26^3 5.03 / 5.06 / 5.15,
+        // 32 x 10 x 102 along z 15.6 / 11.8 / 11.6 (rows in global memory took
+        // twice that on the levels beyond LDS: 46^3 93.6, 32 x 10 x 102 31.6)
+        double best = 0.0;
+        for (int axis = 2; axis >= 1; --axis)
+            for (long k = 1; k <= 16 && k <= d[axis]; ++k) {
+                const long len = (d[axis] + k - 1) / k, items = n / d[axis] * ((d[axis] + len - 1) / len);
+                const long rounds = (items + 1023) / 1024;
+                const double cost = (2.0 * items / 1024.0 + rounds) * (len + 2);
+                if (best > 0.0 && cost >= best) continue;
+                best = cost;
+                p.axis = axis;
+                p.len = (int)len;
+                p.work = (size_t)rounds * len * 1024 * 7;
+            }
+        if (p.lds > kBottomLds) p.lds = 0;
+        return pick(BottomPlan::WIDE, 0, p.work + (p.lds ? 0 : n));
+    } else {
+        const bool cell = Rows::NS == 7;
+        if (n <= 1024) return pick(BottomPlan::REG2, 2, 0);
+        if (n <= 2048 && cell) return pick(BottomPlan::REG4, 4, 0);
+        if (n <= 2048) return pick(BottomPlan::ROWS2, 2, (size_t)Rows::NS * n);
+        if (n <= 4096) return pick(BottomPlan::ROWS4, 4, (size_t)Rows::NS * n);
+        if (p.lds > kBottomLds) p.lds = 0;
+        return pick(BottomPlan::ROWS, 0, (size_t)(Rows::NS + 7) * n);
+    }
+}
 
 // large dynamic LDS is announced once, outside any stream capture
 template <class Rows, class T>
-struct BottomCols {
-    static void prepare() {}
-};
-template <class TS, class T>
-struct BottomCols<NodalRows<TS>, T> {
-    static void prepare() {
-        (void)hipFuncSetAttribute((const void*)bottom_cols_kernel<TS, T, 4>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)kBottomLds);
-        (void)hipFuncSetAttribute((const void*)bottom_cols_kernel<TS, T, 8>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)kBottomLds);
-        (void)hipFuncSetAttribute((const void*)bottom_wide_kernel<TS, T>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)kBottomLds);
-    }
-};
-template <class Rows, class T>
 void bottom_prepare() {
     static const bool once = [] {
-        BottomCols<Rows, T>::prepare();
-        (void)hipFuncSetAttribute((const void*)bottom_kernel<Rows, T, 0, false, 1024, true>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)kBottomLds);
+        const auto lds = [](const void* f) {
+            (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kBottomLds);
+        };
+        if constexpr (Rows::kNodal) {
+            lds((const void*)bottom_cols_kernel<T, T, 4>);
+            lds((const void*)bottom_cols_kernel<T, T, 8>);
+            lds((const void*)bottom_wide_kernel<T, T, true>);
+        } else {
+            lds((const void*)bottom_kernel<Rows, T, 0, false, 1024, true>);
+        }
         return true;
     }();
     (void)once;
 }
 
-// The column variant, when 512 threads hold the level at NPT nodes each along
-// some axis (the first axis that does).
-template <class TS, class T, int NPT>
-inline bool bottom_launch_cols(const NodalRows<TS>& op, long n, const T* b_in, T* x_out,
-                               const BottomArgs& a, hipStream_t s) {
-    const size_t lds = n * sizeof(double) + (size_t)op.g.sg[0] * op.g.sg[1] * op.g.sg[2] * sizeof(TS);
-    if (lds > kBottomLds) return false;
-    for (int axis = 2; axis >= 0; --axis) {
-        const long threads = n / op.g.nn[axis] * ((op.g.nn[axis] + NPT - 1) / NPT);
-        if (threads > 512) continue;
-        bottom_cols_kernel<TS, T, NPT><<<1, (unsigned)((threads + 63) / 64 * 64), lds, s>>>(
-            op, axis, b_in, x_out, a);
-        return true;
-    }
-    return false;
-}
 template <class Rows, class T>
-inline bool bottom_launch_any_cols(const Rows&, long, const T*, T*, const BottomArgs&, hipStream_t) {
-    return false;
-}
-template <class TS, class T>
-inline bool bottom_launch_any_cols(const NodalRows<TS>& op, long n, const T* b_in, T* x_out,
-                                   const BottomArgs& a, hipStream_t s) {
-    if (bottom_launch_cols<TS, T, 4>(op, n, b_in, x_out, a, s) ||
-        bottom_launch_cols<TS, T, 8>(op, n, b_in, x_out, a, s))
-        return true;
-    if (n <= 4096 || n * sizeof(double) > kBottomLds) return false;
-    int axis = 2;
-    for (int d = 1; d >= 0; --d)
-        if (op.g.nn[d] < op.g.nn[axis]) axis = d;
-    bottom_wide_kernel<TS, T><<<1, 1024, n * sizeof(double), s>>>(op, axis, b_in, x_out, a);
-    return true;
-}
-
-// Variants by the number of unknowns n, from what a CU's register file holds
-// (512 threads get 256 VGPRs each, 1024 threads 128): vectors 14 VGPRs, 27-point
-// rows 54 and 7-point rows 14 VGPRs per unknown.  Rows read from global memory
-// took the 1280-node nodal solve 740 us, columns 150; with spilled rows 8 nodes
-// per column thread took 1900 us at 2275 nodes, without 527.
-template <class Rows, class T>
-void bottom_launch(const Rows& op, long n, const T* b_in, T* x_out, const BottomArgs& a,
-                          hipStream_t s) {
-    const size_t lds = (size_t)n * sizeof(double);
-    const auto up64 = [](long v) { return (unsigned)((v + 63) / 64 * 64); };
-    if (n <= 512)
-        bottom_kernel<Rows, T, 1, true, 512, true><<<1, up64(n), lds, s>>>(op, b_in, x_out, a);
-    else if (bottom_launch_any_cols(op, n, b_in, x_out, a, s))
+void bottom_launch(const Rows& op, const T* b_in, T* x_out, const BottomArgs& a, hipStream_t s) {
+    const BottomPlan p = bottom_plan(op);
+    if (p.kind == BottomPlan::REG1) {
+        bottom_kernel<Rows, T, 1, true, 512, true><<<1, p.threads, p.lds, s>>>(op, b_in, x_out, a);
         return;
-    else if (n <= 1024)
-        bottom_kernel<Rows, T, 2, true, 512, true><<<1, up64((n + 1) / 2), lds, s>>>(op, b_in, x_out, a);
-    else if (n <= 2048 && Rows::NS == 7)
-        bottom_kernel<Rows, T, Rows::NS == 7 ? 4 : 1, true, 512, true><<<1, up64((n + 3) / 4), lds, s>>>(op, b_in, x_out, a);
-    else if (n <= 2048)
-        bottom_kernel<Rows, T, 2, false, 1024, true><<<1, up64((n + 1) / 2), lds, s>>>(op, b_in, x_out, a);
-    else if (n <= 4096)
-        bottom_kernel<Rows, T, 4, false, 1024, true><<<1, up64((n + 3) / 4), lds, s>>>(op, b_in, x_out, a);
-    else if (lds <= kBottomLds)
-        bottom_kernel<Rows, T, 0, false, 1024, true><<<1, 1024, lds, s>>>(op, b_in, x_out, a);
-    else
-        bottom_kernel<Rows, T, 0, false, 1024, false><<<1, 1024, 0, s>>>(op, b_in, x_out, a);
+    }
+    if constexpr (Rows::kNodal) {
+        if (p.kind == BottomPlan::COLS4)
+            bottom_cols_kernel<T, T, 4><<<1, p.threads, p.lds, s>>>(op, p.axis, b_in, x_out, a);
+        else if (p.kind == BottomPlan::COLS8)
+            bottom_cols_kernel<T, T, 8><<<1, p.threads, p.lds, s>>>(op, p.axis, b_in, x_out, a);
+        else if (p.kind == BottomPlan::ROWS4)
+            bottom_kernel<Rows, T, 4, false, 1024, true><<<1, p.threads, p.lds, s>>>(op, b_in, x_out, a);
+        else if (p.lds > 0)
+            bottom_wide_kernel<T, T, true><<<1, p.threads, p.lds, s>>>(op, p.axis, p.len, b_in, x_out, a);
+        else
+            bottom_wide_kernel<T, T, false><<<1, p.threads, 0, s>>>(op, p.axis, p.len, b_in, x_out, a);
+    } else {
+        if (p.kind == BottomPlan::REG2)
+            bottom_kernel<Rows, T, 2, true, 512, true><<<1, p.threads, p.lds, s>>>(op, b_in, x_out, a);
+        else if (p.kind == BottomPlan::REG4)
+            bottom_kernel<Rows, T, Rows::NS == 7 ? 4 : 1, true, 512, true><<<1, p.threads, p.lds, s>>>(op, b_in, x_out, a);
+        else if (p.kind == BottomPlan::ROWS2)
+            bottom_kernel<Rows, T, 2, false, 1024, true><<<1, p.threads, p.lds, s>>>(op, b_in, x_out, a);
+        else if (p.kind == BottomPlan::ROWS4)
+            bottom_kernel<Rows, T, 4, false, 1024, true><<<1, p.threads, p.lds, s>>>(op, b_in, x_out, a);
+        else if (p.lds > 0)
+            bottom_kernel<Rows, T, 0, false, 1024, true><<<1, p.threads, p.lds, s>>>(op, b_in, x_out, a);
+        else
+            bottom_kernel<Rows, T, 0, false, 1024, false><<<1, p.threads, 0, s>>>(op, b_in, x_out, a);
+    }
 }
 
 // instantiated in bottom_nodal.hip and bottom_cell.hip
 #define MGX_BOTTOM_INSTANCE(EXT, ROWS, T)                                                            \
     EXT template void bottom_prepare<ROWS, T>();                                                     \
-    EXT template void bottom_launch<ROWS, T>(const ROWS&, long, const T*, T*, const BottomArgs&, hipStream_t)
+    EXT template void bottom_launch<ROWS, T>(const ROWS&, const T*, T*, const BottomArgs&, hipStream_t)
 MGX_BOTTOM_INSTANCE(extern, NodalRows<float>, float);
 MGX_BOTTOM_INSTANCE(extern, NodalRows<double>, double);
 

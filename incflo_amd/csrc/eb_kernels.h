@@ -78,9 +78,9 @@ __device__ inline double eb_apply_node(const EBLev& L, const double* x, int i, i
 // The rows of the EB operator, for the row tables and the bottom solve: inactive nodes are held at zero.
 struct EBRows {
     static constexpr int NS = 27;
-    static constexpr bool kRedBlack = false;
+    static constexpr bool kRedBlack = false, kNodal = false;
     EBLev L;
-    __device__ int dim(int d) const { return L.g.nn[d]; }
+    __host__ __device__ int dim(int d) const { return L.g.nn[d]; }
     __device__ int per(int d) const { return L.g.per[d]; }
     __device__ bool row(int id, int i, int j, int k, double (&C)[NS]) const {
         const KGeom& g = L.g;

@@ -475,7 +475,7 @@ void EBNodal::setup(const NodalGeom& g0, int nlev, const std::vector<int>& type,
         lv.x = lv.x_buf.as<double>();
         lv.x2 = lv.x2_buf.as<double>();
     }
-    bottom_work.alloc(bottom_work_doubles(L.back().g.nnode(), 27) * sizeof(double));
+    bottom_work.alloc(std::max<size_t>(1, bottom_plan(EBRows{lev(nlev - 1)}).work) * sizeof(double));
     bottom_prepare<EBRows, double>();
     ready = true;
 }
@@ -590,7 +590,7 @@ void EBNodal::vcycle(const MGOpts& o, bool first, hipStream_t s) {
         ba.rtol = o.bottom_rtol;
         ba.omega = nodal_omega(lb.g, o.omega);
         ba.singular = lb.g.singular() ? 1 : 0;
-        bottom_launch<EBRows, double>(EBRows{lev(nl - 1)}, lb.g.nnode(), lb.b_buf.as<double>(),
+        bottom_launch<EBRows, double>(EBRows{lev(nl - 1)}, lb.b_buf.as<double>(),
                                       lb.x, ba, s);
     }
     for (int l = nl - 2; l >= 0; --l) {

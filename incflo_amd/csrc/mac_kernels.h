@@ -330,11 +330,11 @@ static __global__ void mac_beta_from_rho_kernel(MGeomK g, int d, const double* _
 template <class T>
 struct MacRows {
     static constexpr int NS = 7;
-    static constexpr bool kRedBlack = true;
+    static constexpr bool kRedBlack = true, kNodal = false;
     MGeomK g;
     MCoef<double> c;
     const T *bx, *by, *bz, *a;
-    __device__ int dim(int d) const { return g.n[d]; }
+    __host__ __device__ int dim(int d) const { return g.n[d]; }
     __device__ int per(int d) const { return g.per[d]; }
     __device__ bool row(int id, int i, int j, int k, double (&C)[NS]) const {
         const int p[3] = {i, j, k};

@@ -58,7 +58,13 @@ void MacHierarchy<T>::build(const MacGeom& g0, int nlev, int few) {
         lv.x2 = lv.x2_buf.template as<T>();
         lv.r = lv.r_buf.template as<T>();
     }
-    bottom_work.alloc(bottom_work_doubles(L[(few ? few : nlev) - 1].g.ncell(), 7) * sizeof(double));
+    size_t work = 1;
+    for (int l = (few ? few : nlev) - 1; l < nlev; ++l) {
+        MacRows<T> bottom{};
+        bottom.g = L[l].kg;
+        work = std::max(work, bottom_plan(bottom).work);
+    }
+    bottom_work.alloc(work * sizeof(double));
     used = nlev;
     bottom_prepare<MacRows<T>, T>();
     built = true;
@@ -233,7 +239,7 @@ void MacHierarchy<T>::vcycle_body(const MGOpts& o, hipStream_t s, int* bottom_it
         ba.singular = lb.g.singular() ? 1 : 0;
         ba.iters_acc = bottom_iters;
         const MacRows<T> rows{lb.kg, make_mcoef<double>(lb.g.dx), lb.beta[0], lb.beta[1], lb.beta[2], lb.a};
-        bottom_launch<MacRows<T>, T>(rows, lb.g.ncell(), lb.b, lb.x, ba, s);
+        bottom_launch<MacRows<T>, T>(rows, lb.b, lb.x, ba, s);
     }
     x0_guess = false;
     if (lc < nl - 1) mac_coarse_cycle_kernel<T><<<1, 1024, 0, s>>>(mac_coarse_args(L, nl, lc, o, 1));

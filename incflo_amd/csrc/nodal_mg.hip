@@ -433,7 +433,17 @@ void NodalHierarchy<T>::build(const NodalGeom& g0, int nlev, int few) {
         lv.x2 = lv.x2_buf.template as<T>();
         lv.r = lv.r_buf.template as<T>();
     }
-    bottom_work.alloc(bottom_work_doubles(L[(few ? few : nlev) - 1].g.nnode(), 27) * sizeof(double));
+    size_t work = 1;
+    for (int l = (few ? few : nlev) - 1; l < nlev; ++l) {
+        NodalRows<T> bottom{};
+        bottom.g = L[l].kg;
+        const size_t nb = L[l].g.nnode();
+        work = std::max(work, bottom_plan(bottom).work);
+        // the rows and vectors of a bottom that the tuning table folds into the
+        // coarse levels' workgroup (its multiplied vector fits LDS)
+        if (nb * sizeof(double) <= kBottomLds) work = std::max(work, 34 * nb);
+    }
+    bottom_work.alloc(work * sizeof(double));
     used = nlev;
     built = true;
 }
@@ -660,7 +670,7 @@ void NodalHierarchy<T>::vcycle_body(const MGOpts& o, hipStream_t s, int* bottom_
     ba.iters_acc = bottom_iters;
     if (lc == nl - 1) {
         const NodalRows<T> rows{lb.kg, make_coef<double>(lb.g.dx), lb.sig, mask(nl - 1)};
-        bottom_launch<NodalRows<T>, T>(rows, lb.g.nnode(), lb.b, lb.x, ba, s);
+        bottom_launch<NodalRows<T>, T>(rows, lb.b, lb.x, ba, s);
     } else {
         CoarseArgs<T> ca{};
         ca.nl = nl - lc;

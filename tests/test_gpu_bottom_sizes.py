@@ -1,7 +1,9 @@
 """GPU tests of the bottom-solve kernels at the sizes where their variant
-changes (rows in registers up to 512 unknowns, columns up to 4096 nodes, rows
-in global memory, the multiplied vector in LDS or global memory) and of the
-extra coarsening of large bottoms.
+changes: nodal rows in registers up to 512 nodes, columns of 4 or 8 nodes where
+512 threads hold the level, rows in global memory for others up to 4096, then
+segments of columns (the multiplied vector in LDS or global memory); EB and
+cell-centred rows in registers up to 1024 and 2048 unknowns, in global memory
+above, and their vectors from 4096 on.
 
 max_coarsening_level 0 makes the whole level the bottom, so each size runs one
 variant.  The check is the answer's residual under the oracle's FP64 operator:
@@ -43,16 +45,22 @@ NODAL = [  # cells, periodicity, lo, hi, kind, overset mask
     ((15, 9, 7), (0, 0, 0), (INF, N, N), (D, N, N), "bicgcg", False),      # 1280
     ((17, 15, 13), (1, 1, 1), (0, 0, 0), (0, 0, 0), "bicgcg", False),      # 3315: 8 per thread
     ((15, 15, 15), (0, 0, 0), (D, N, N), (N, N, N), "cg", True),           # 4096
-    ((21, 19, 17), (0, 1, 0), (N, 0, D), (D, 0, N), "bicgcg", False),      # 7480: whole columns
+    ((12, 25, 9), (0, 0, 0), (INF, N, N), (D, N, N), "bicgcg", False),     # 3380: rows in memory
+    ((10, 19, 18), (1, 0, 1), (0, N, 0), (0, D, 0), "cg", True),           # 3600
+    ((10, 18, 17), (0, 0, 0), (N, N, N), (N, N, N), "bicgcg", False),      # 3762
+    ((21, 19, 17), (0, 1, 0), (N, 0, D), (D, 0, N), "bicgcg", False),      # 7480: segments
     ((20, 4, 60), (0, 0, 1), (D, N, 0), (N, N, 0), "cg", True),            # 6300, columns along y
     ((30, 27, 25), (1, 1, 1), (0, 0, 0), (0, 0, 0), "bicgcg", False),      # 20250: beyond LDS
+    ((32, 29, 23), (0, 0, 0), (INF, N, N), (D, N, N), "cg", True),         # 23760
+    ((3, 130, 45), (1, 0, 0), (0, N, N), (0, D, N), "bicgcg", False),      # 18078, in LDS
 ]
 
 
+@pytest.mark.parametrize("mixed", [False, True])
 @pytest.mark.parametrize("n,per,bclo,bchi,kind,masked", NODAL)
-def test_nodal_bottom_of_every_size(ctx, orc, n, per, bclo, bchi, kind, masked):
+def test_nodal_bottom_of_every_size(ctx, orc, n, per, bclo, bchi, kind, masked, mixed):
     from incflo_amd import mgx
-    _say(f"case nodal bottom {n} {kind} mask {masked}")
+    _say(f"case nodal bottom {n} {kind} mask {masked} mixed {mixed}")
     ph = (1.0, 1.3, 0.9)
     g = orc.Geom.make(n, periodic=per, bclo=bclo, bchi=bchi, prob_hi=ph)
     rng = np.random.default_rng(sum(n))
@@ -73,7 +81,7 @@ def test_nodal_bottom_of_every_size(ctx, orc, n, per, bclo, bchi, kind, masked):
         b -= b.mean()
     rd = ctx.array(B.to_boxed(b, bxs, 0, nodal=True, periodic=per))
     xd = ctx.array(B.field_size(bxs, 0, 1, True))
-    info = P.solve(xd, 0, rd, 0, RTOL, mode=mgx.MODE_FP64)
+    info = P.solve(xd, 0, rd, 0, RTOL, mode=mgx.MODE_MIXED if mixed else mgx.MODE_FP64)
     x = B.from_boxed(xd.download(), bxs, 0, g.node_shape(), nodal=True)
     P.close()
     assert info.converged and info.nlevels == 1
@@ -126,11 +134,19 @@ def test_mac_bottom_of_every_size(ctx, orc, n, per, bclo, bchi, kind):
     assert np.max(np.abs(r)) <= 2 * RTOL * np.max(np.abs(b))
 
 
-@pytest.mark.parametrize("levels", [0, 1, 2])  # bottoms of 8976, 1224 and 180 nodes
-def test_eb_bottom_of_every_size(ctx, orc, levels):
+EB = [((32, 16, 16), 0),  # 8976 nodes: rows and vectors in global memory
+      ((32, 16, 16), 1),  # 1224: rows in global memory
+      ((32, 16, 16), 2),  # 180
+      ((16, 8, 6), 0),    # 918: rows of two nodes per thread in registers
+      ((24, 12, 10), 0),  # 3250: rows in global memory, four nodes per thread
+      ((50, 25, 15), 0)]  # 19890: beyond LDS
+
+
+@pytest.mark.parametrize("n,levels", EB)
+def test_eb_bottom_of_every_size(ctx, orc, n, levels):
     from incflo_amd import mgx
-    _say(f"case eb bottom, max_coarsening_level {levels}")
-    n, ph, per, bclo, bchi = (32, 16, 16), (2.0, 1.0, 1.0), (0, 0, 1), (INF, N, 0), (D, N, 0)
+    _say(f"case eb bottom {n}, max_coarsening_level {levels}")
+    ph, per, bclo, bchi = (2.0, 1.0, n[2] / n[1]), (0, 0, 1), (INF, N, 0), (D, N, 0)
     g = orc.Geom.make(n, periodic=per, bclo=bclo, bchi=bchi, prob_hi=ph)
     bxs = B.chop_domain(n, 16)
     P = mgx.NodalProjector(ctx, mgx.make_level(n, bxs, periodic=per, prob_hi=ph))
