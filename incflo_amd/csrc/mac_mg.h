@@ -62,7 +62,7 @@ struct MacLevel {
     T* b = nullptr;
     T* x = nullptr;
     T* x2 = nullptr;  // the iterate between the down and the up leg
-    T* r = nullptr;
+    T* r = nullptr;   // residual, on the levels of the one-workgroup coarse cycle only
 };
 
 template <class T>

@@ -49,14 +49,10 @@ void MacHierarchy<T>::build(const MacGeom& g0, int nlev, int few) {
         }
         if (l > 0) lv.b_buf.alloc(n * sizeof(T));
         lv.x_buf.alloc(n * sizeof(T));
-        if (l < nlev - 1) {
-            lv.x2_buf.alloc(n * sizeof(T));
-            lv.r_buf.alloc(n * sizeof(T));
-        }
+        if (l < nlev - 1) lv.x2_buf.alloc(n * sizeof(T));
         lv.b = lv.b_buf.template as<T>();
         lv.x = lv.x_buf.template as<T>();
         lv.x2 = lv.x2_buf.template as<T>();
-        lv.r = lv.r_buf.template as<T>();
     }
     size_t work = 1;
     for (int l = (few ? few : nlev) - 1; l < nlev; ++l) {
@@ -133,8 +129,25 @@ static bool same_cycle_opts(const MGOpts& a, const MGOpts& b) {
            a.bottom_rtol == b.bottom_rtol && a.bottom_solver == b.bottom_solver;
 }
 
+// the first level of the one-workgroup coarse cycle of a V-cycle of nl levels
+// (nl - 1: none)
+template <class T>
+static int mac_coarse_first(const std::vector<MacLevel<T>>& L, int nl) {
+    const long maxc = mac_coarse_cells();
+    int lc = nl - 1;
+    while (lc - 1 >= 1 && L[lc - 1].g.ncell() <= maxc && nl - 1 - (lc - 1) <= kMacCoarseMax) --lc;
+    return lc;
+}
+
 template <class T>
 void MacHierarchy<T>::vcycle(const MGOpts& o, hipStream_t s, int* bottom_iters) {
+    // residuals of the levels of that cycle, which the tuning table may change;
+    // the tile kernels keep theirs in LDS
+    for (int l = mac_coarse_first(L, used); l < used - 1; ++l)
+        if (!L[l].r) {
+            L[l].r_buf.alloc(L[l].g.ncell() * sizeof(T));
+            L[l].r = L[l].r_buf.template as<T>();
+        }
     if (!graphs) {
         vcycle_body(o, s, bottom_iters);
         return;
@@ -187,16 +200,6 @@ void MacHierarchy<T>::vcycle(const MGOpts& o, hipStream_t s, int* bottom_iters) 
 }
 
 static_assert(sizeof(MacCoarseArgs<double>) <= 3072, "coarse-cycle kernel arguments");
-
-// the first level of the one-workgroup coarse cycle of a V-cycle of nl levels
-// (nl - 1: none)
-template <class T>
-static int mac_coarse_first(const std::vector<MacLevel<T>>& L, int nl) {
-    const long maxc = mac_coarse_cells();
-    int lc = nl - 1;
-    while (lc - 1 >= 1 && L[lc - 1].g.ncell() <= maxc && nl - 1 - (lc - 1) <= kMacCoarseMax) --lc;
-    return lc;
-}
 
 template <class T>
 static MacCoarseArgs<T> mac_coarse_args(std::vector<MacLevel<T>>& L, int nl, int lc, const MGOpts& o,
