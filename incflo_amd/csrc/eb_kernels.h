@@ -123,7 +123,7 @@ static __global__ void __launch_bounds__(256) eb_apply_kernel(EBLev L, const dou
 // (27 coefficients, one array per neighbour, so every load is coalesced over
 // the rows); the other active nodes see regular cells only and are swept by
 // the plain nodal stencil kernel, with the nodes listed here as type 2.  A
-// level of at most kEBRowNodes nodes has all its rows in the table and takes
+// level of at most eb_row_nodes() nodes has all its rows in the table and takes
 // one launch per pass: below that size the two launches of the split cost
 // more than reading the 27 coefficients.
 struct EBRowArgs {

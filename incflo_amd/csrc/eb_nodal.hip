@@ -355,17 +355,11 @@ void upload(DevBuf& buf, const std::vector<T>& h) {
     if (!h.empty()) MGX_HIP(hipMemcpy(buf.p, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
 }
 
-// Levels of at most this many nodes have all their rows in the table.  A
-// projection pair of 256x64x64 cells took 8.29 ms with the 257x65x64 level split
-// and the 129x33x32 one in the table, 8.51 ms with both split, 10.8 ms with both
-// in the table.
-constexpr long kEBRowNodes = 200000;
-
 // the rows that the level's table holds (a node's cells: mask_h is up to date)
 void row_nodes(EBLevelData& lv) {
     const NodalGeom& g = lv.g;
     const long nn = g.nnode();
-    lv.all_rows = nn <= kEBRowNodes;
+    lv.all_rows = nn <= eb_row_nodes();
     lv.nrow = (int)nn;
     if (!lv.all_rows) {
         std::vector<unsigned char> type(lv.mask_h);

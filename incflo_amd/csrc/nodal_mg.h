@@ -147,6 +147,10 @@ class TileSet {
 // one-workgroup coarse cycle takes (tuning table mac_coarse_cells; 0: none)
 long mac_coarse_cells();
 
+// nodes up to which an embedded-boundary level has all its rows in the table
+// (tuning table eb_row_nodes)
+long eb_row_nodes();
+
 // Full weighting of a fine level's nodal array onto every node of the level
 // below it (dense, z-streamed as the V-cycle's restriction; Dirichlet nodes 0)
 template <class T>

@@ -90,6 +90,17 @@ static int g_amr_tile_width = 16;
 static int g_amr_tile_width32 = 64;
 static int g_amr_tile_kz = TileSet::kKZ;
 
+// embedded-boundary levels of at most this many nodes have all their rows in the
+// table (read when a handle is set up).  A projection pair of 256x64x64 cells took
+// 8.29 ms with the 257x65x64 level split and the 129x33x32 one in the table, 8.51 ms
+// with both split, 10.8 ms with both in the table.
+static long g_eb_row_nodes = 200000;
+
+long eb_row_nodes() {
+    std::lock_guard<std::mutex> lk(g_tune_mtx);
+    return g_eb_row_nodes;
+}
+
 long mac_coarse_cells() {
     std::lock_guard<std::mutex> lk(g_tune_mtx);
     return g_mac_coarse_cells;
@@ -1189,6 +1200,7 @@ std::string tuning_table() {
     o << "amr_tile_width " << g_amr_tile_width << "\n";
     o << "amr_tile_width32 " << g_amr_tile_width32 << "\n";
     o << "amr_tile_kz " << g_amr_tile_kz << "\n";
+    o << "eb_row_nodes " << g_eb_row_nodes << "\n";
     return o.str();
 }
 
@@ -1196,7 +1208,7 @@ void set_tuning_table(const std::string& text) {
     std::istringstream in(text);
     std::string tag;
     std::map<ShapeKey, StencilShape> shapes;
-    long coarse = 1, mac_coarse = 512;
+    long coarse = 1, mac_coarse = 512, eb_rows = 200000;
     int pairs = 0, tilew = 16, tilew32 = 64, tilekz = TileSet::kKZ;
     while (in >> tag) {
         if (tag == "stencil") {
@@ -1228,6 +1240,9 @@ void set_tuning_table(const std::string& text) {
         } else if (tag == "mac_coarse_cells") {
             in >> mac_coarse;
             MGX_REQUIRE(!in.fail() && mac_coarse >= 0, MGX_ERR_ARG, "tuning table: bad mac_coarse_cells");
+        } else if (tag == "eb_row_nodes") {
+            in >> eb_rows;
+            MGX_REQUIRE(!in.fail() && eb_rows >= 0, MGX_ERR_ARG, "tuning table: bad eb_row_nodes");
         } else if (tag == "jacobi_pairs") {
             in >> pairs;
             MGX_REQUIRE(!in.fail() && (pairs == 0 || pairs == 1), MGX_ERR_ARG,
@@ -1240,6 +1255,7 @@ void set_tuning_table(const std::string& text) {
     g_shapes = std::move(shapes);
     g_coarse_nodes = coarse;
     g_mac_coarse_cells = mac_coarse;
+    g_eb_row_nodes = eb_rows;
     g_jacobi_pairs = pairs;
     g_amr_tile_width = tilew;
     g_amr_tile_width32 = tilew32;

@@ -231,7 +231,9 @@ MGX_API int mgx_nodal_autotune(mgx_nodal h, int mode, char* report, int report_l
  * fine levels' stencil tiles "amr_tile_width 16|64" (FP64),
  * "amr_tile_width32 16|64" (FP32) and "amr_tile_kz K" planes, and
  * "mac_coarse_cells N": cell-centred multigrid levels below the first with
- * at most N cells run in one workgroup per V-cycle half, 0: none), for caching
+ * at most N cells run in one workgroup per V-cycle half, 0: none;
+ * "eb_row_nodes N": embedded-boundary levels of at most N nodes are swept from
+ * assembled rows alone, on handles set up later), for caching
  * per device model; mgx_tuning_set loads such a text (replacing the table;
  * lines left out take their defaults). */
 MGX_API int mgx_tuning_get(char* buf, int len);
