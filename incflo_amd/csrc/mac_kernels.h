@@ -91,6 +91,22 @@ __device__ __forceinline__ T mac_apply_cell(const MGeomK& g, const MCoef<T>& c, 
     return acc;
 }
 
+// One colour of red-black Gauss-Seidel, in place.  Threads cover pairs of cells
+// along x; each updates the cell of the requested colour.
+template <class T>
+static __global__ void mac_gsrb_kernel(MGeomK g, MCoef<T> c, const T* __restrict__ bx,
+                                       const T* __restrict__ by, const T* __restrict__ bz,
+                                       const T* __restrict__ a, const T* __restrict__ b, T* x, int color) {
+    int ih, j, k;
+    if (!grid_point((g.n[0] + 1) / 2, g.n[1], ih, j, k)) return;
+    const int i = 2 * ih + ((j + k + color) & 1);
+    if (i >= g.n[0]) return;
+    T dg;
+    const T acc = mac_apply_cell<T, T, T>(g, c, bx, by, bz, a, x, i, j, k, dg);
+    const long id = cidx(g, i, j, k);
+    if (dg != (T)0) x[id] += (b[id] - acc) / dg;
+}
+
 enum { MK_RESID = 0, MK_UPDRES = 1, MK_APPLY = 2 };
 
 // RESID: r = b - L x.  UPDRES: x_out = x + cor, r = b - L x_out.  APPLY: r = L x.
@@ -143,6 +159,15 @@ static __global__ void mac_restrict_kernel(MGeomK gf, MGeomK gc, const T* __rest
     rc[cidx(gc, I, J, K)] = (T)0.125 * s;
 }
 
+// piecewise-constant prolongation added onto the fine correction
+template <class T>
+static __global__ void mac_prolong_add_kernel(MGeomK gf, MGeomK gc, const T* __restrict__ xc,
+                                              T* __restrict__ xf) {
+    int i, j, k;
+    if (!grid_point(gf.n[0], gf.n[1], i, j, k)) return;
+    xf[cidx(gf, i, j, k)] += xc[cidx(gc, i >> 1, j >> 1, k >> 1)];
+}
+
 // The coarse levels of a V-cycle in one workgroup (each level at most a few
 // thousand cells, where separate launches would each cost more than their
 // work): L[0..nlev-1] are smoothed, L[nlev] is the level below them (the
@@ -150,7 +175,7 @@ static __global__ void mac_restrict_kernel(MGeomK gf, MGeomK gc, const T* __rest
 // Gauss-Seidel, r = b - L x, then the next level's b = the mean of 8 r.  Up:
 // from the deepest, x += the parent's x, nu2 x (red, black).  The per-cell
 // arithmetic is that of the tile kernels (mac_tile_kernels.h), with a
-// workgroup barrier between passes, so the results are the same bit for bit.
+// workgroup barrier between passes, and the results are the same bit for bit.
 constexpr int kMacCoarseMax = 8;
 
 template <class T>

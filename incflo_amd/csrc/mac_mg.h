@@ -62,7 +62,7 @@ struct MacLevel {
     T* b = nullptr;
     T* x = nullptr;
     T* x2 = nullptr;  // the iterate between the down and the up leg
-    T* r = nullptr;   // residual, on the levels of the one-workgroup coarse cycle only
+    T* r = nullptr;   // residual, on levels that are not smoothed on tiles
 };
 
 template <class T>
@@ -103,7 +103,8 @@ class MacHierarchy {
         const T* b0;
         bool guess0;
         int* bottom_iters;
-        long coarse;  // mac_coarse_cells() at capture
+        long coarse;  // mac_coarse_cells() and mac_tiles() at capture
+        MacTiles tiles;
         int used;
         MGOpts o;
         hipGraphExec_t exec;

@@ -106,6 +106,18 @@ void MacHierarchy<T>::set_acoef(const double* a0, hipStream_t s) {
     }
 }
 
+template <class T>
+static bool by_colours(const MacLevel<T>& lv, const MacTiles& tiles) {
+    return sizeof(T) == 4 && lv.g.n[0] % 32 == 0 && lv.g.ncell() > tiles.max;
+}
+
+template <class T>
+static void gsrb(MacLevel<T>& lv, hipStream_t s) {
+    for (int color = 0; color < 2; ++color)
+        mac_gsrb_kernel<T><<<grid3((lv.g.n[0] + 1) / 2, lv.g.n[1], lv.g.n[2]), block3(), 0, s>>>(
+            lv.kg, lv.c, lv.beta[0], lv.beta[1], lv.beta[2], lv.a, lv.b, lv.x, color);
+}
+
 // the level's part of the tile kernels' arguments (w: the level below, or v)
 template <class T>
 static MacTileArgs<T> mac_tile_args(const MacLevel<T>& v, const MacLevel<T>& w) {
@@ -141,10 +153,12 @@ static int mac_coarse_first(const std::vector<MacLevel<T>>& L, int nl) {
 
 template <class T>
 void MacHierarchy<T>::vcycle(const MGOpts& o, hipStream_t s, int* bottom_iters) {
-    // residuals of the levels of that cycle, which the tuning table may change;
-    // the tile kernels keep theirs in LDS
-    for (int l = mac_coarse_first(L, used); l < used - 1; ++l)
-        if (!L[l].r) {
+    // residuals of the levels that are not smoothed on tiles (these keep theirs in
+    // LDS); the tuning table may change which
+    const MacTiles tiles = mac_tiles();
+    const int lc = mac_coarse_first(L, used);
+    for (int l = 0; l < used - 1; ++l)
+        if (!L[l].r && (l >= lc || by_colours(L[l], tiles))) {
             L[l].r_buf.alloc(L[l].g.ncell() * sizeof(T));
             L[l].r = L[l].r_buf.template as<T>();
         }
@@ -157,7 +171,7 @@ void MacHierarchy<T>::vcycle(const MGOpts& o, hipStream_t s, int* bottom_iters) 
     const CycleGraph* hit = nullptr;
     for (const CycleGraph& c : cache_)
         if (c.x0 == L[0].x && c.b0 == L[0].b && c.guess0 == guess0 && c.bottom_iters == bottom_iters &&
-            c.coarse == coarse && c.used == used && same_cycle_opts(c.o, o))
+            c.coarse == coarse && c.tiles == tiles && c.used == used && same_cycle_opts(c.o, o))
             hit = &c;
     if (!hit) {
         if (cache_.size() >= 16) drop_graphs();
@@ -180,7 +194,7 @@ void MacHierarchy<T>::vcycle(const MGOpts& o, hipStream_t s, int* bottom_iters) 
             if (e == hipSuccess && body_ok) e = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
             if (g) (void)hipGraphDestroy(g);
             if (e == hipSuccess && body_ok) {
-                cache_.push_back(CycleGraph{L[0].x, L[0].b, guess0, bottom_iters, coarse, used, o, exec});
+                cache_.push_back(CycleGraph{L[0].x, L[0].b, guess0, bottom_iters, coarse, tiles, used, o, exec});
                 hit = &cache_.back();
             } else {
                 ok = false;
@@ -227,10 +241,25 @@ void MacHierarchy<T>::vcycle_body(const MGOpts& o, hipStream_t s, int* bottom_it
     const int nl = used;
     // levels lc..nl-2 in one workgroup (lc == nl - 1: none)
     const int lc = mac_coarse_first(L, nl);
-    // down: x (a guess on level 0) -> x2; up: x2 -> x
-    for (int l = 0; l < lc; ++l)
-        mac_tile_sweeps(mac_tile_args(L[l], L[l + 1]), l == 0 && x0_guess ? MT_X : MT_ZERO, L[l].x, L[l].x2,
-                        o.nu1, true, s);
+    const MacTiles tiles = mac_tiles();
+    int down, up;
+    mac_leg_launches(o.nu1, o.nu2, down, up);
+    // down from x (a guess on level 0), up into x
+    for (int l = 0; l < lc; ++l) {
+        MacLevel<T>& lv = L[l];
+        MacLevel<T>& cv = L[l + 1];
+        const bool guess = l == 0 && x0_guess;
+        if (!by_colours(lv, tiles)) {
+            mac_tile_sweeps(mac_tile_args(lv, cv), guess ? MT_X : MT_ZERO, lv.x, lv.x2, o.nu1, down, true,
+                            tiles, s);
+            continue;
+        }
+        if (!guess) zero_kernel<T><<<grid1d(lv.g.ncell()), 256, 0, s>>>(lv.x, lv.g.ncell());
+        for (int q = 0; q < o.nu1; ++q) gsrb(lv, s);
+        mac_resid_kernel<T, T, MK_RESID><<<grid3(lv.g.n[0], lv.g.n[1], lv.g.n[2]), block3(), 0, s>>>(
+            lv.kg, lv.c, lv.beta[0], lv.beta[1], lv.beta[2], lv.a, lv.b, lv.x, nullptr, nullptr, lv.r, nullptr);
+        mac_restrict_kernel<T><<<grid3(cv.g.n[0], cv.g.n[1], cv.g.n[2]), block3(), 0, s>>>(lv.kg, cv.kg, lv.r, cv.b);
+    }
     if (lc < nl - 1) mac_coarse_cycle_kernel<T><<<1, 1024, 0, s>>>(mac_coarse_args(L, nl, lc, o, 0));
     {
         MacLevel<T>& lb = L[nl - 1];
@@ -246,8 +275,18 @@ void MacHierarchy<T>::vcycle_body(const MGOpts& o, hipStream_t s, int* bottom_it
     }
     x0_guess = false;
     if (lc < nl - 1) mac_coarse_cycle_kernel<T><<<1, 1024, 0, s>>>(mac_coarse_args(L, nl, lc, o, 1));
-    for (int l = lc - 1; l >= 0; --l)
-        mac_tile_sweeps(mac_tile_args(L[l], L[l + 1]), MT_PROLONG, L[l].x2, L[l].x, o.nu2, false, s);
+    for (int l = lc - 1; l >= 0; --l) {
+        MacLevel<T>& lv = L[l];
+        if (!by_colours(lv, tiles)) {
+            T* from = down % 2 ? lv.x2 : lv.x;
+            mac_tile_sweeps(mac_tile_args(lv, L[l + 1]), MT_PROLONG, from, from == lv.x ? lv.x2 : lv.x, o.nu2,
+                            up, false, tiles, s);
+            continue;
+        }
+        mac_prolong_add_kernel<T><<<grid3(lv.g.n[0], lv.g.n[1], lv.g.n[2]), block3(), 0, s>>>(
+            lv.kg, L[l + 1].kg, L[l + 1].x, lv.x);
+        for (int q = 0; q < o.nu2; ++q) gsrb(lv, s);
+    }
 }
 
 template class MacHierarchy<double>;

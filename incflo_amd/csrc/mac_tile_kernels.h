@@ -10,8 +10,8 @@
 // shrinks by one cell per colour, recomputed by each tile), forms the residual
 // and restricts it, and writes x and the coarse right-hand side once.  b and the
 // coefficients come from the caches for each update (x 2-3 per cell).  The
-// per-cell arithmetic and its order are those of one launch per colour, so the
-// results are the same bit for bit.
+// per-cell arithmetic and its order are those of one launch per colour, and the
+// results are the same bit for bit, whichever tiles a level takes.
 //   8 x 8 x 8 tiles: many workgroups with short stages (small levels);
 //   16 x 16 x 8 tiles: 2.05 updates per cell and sweep pair instead of 4.2.
 // Bound by the latency of the stages (5 barriers) on small levels, by the L2
@@ -19,6 +19,7 @@
 #pragma once
 
 #include "mac_kernels.h"
+#include "nodal_mg.h"
 
 namespace mgx {
 
@@ -115,7 +116,7 @@ static __global__ void __launch_bounds__(512) mac_tile_kernel(MacTileArgs<T> a) 
     __shared__ int px[LX], py[LY], pz[LZ];  // domain indices of the tile's columns, -1 outside
     const MGeomK& g = a.g;
     const int tid = threadIdx.x;
-    const int lb = xcd_remap(blockIdx.x, a.gx * a.gy * a.gz);
+    const int lb = xcd_order(blockIdx.x, a.gx * a.gy * a.gz, 4096);
     const int x0 = TX * (lb % a.gx), y0 = TY * ((lb / a.gx) % a.gy), z0 = TZ * (lb / (a.gx * a.gy));
     auto fill = [&](int* p, int len, int o, int d) {
         for (int e = tid; e < len; e += NT) {
@@ -336,21 +337,12 @@ static __global__ void __launch_bounds__(512) mac_reg_tile_kernel(MacTileArgs<T>
     }
 }
 
-// Levels of at most kMacRegTile cells (one 8 x 8 x 8 tile per CU) take the
-// register tiles, up to kMacBigTile 8 x 8 x 8 tiles, larger ones 16 x 16 x 8.
-// Per leg (down / up, FP64): 48 x 32 x 24 cells 11 / 11.6 us with registers, 16 / 13
-// without; 96 x 64 x 48 cells 35 / 35 with, 28 / 23 without (one launch per colour
-// took 49 / 38); 128^3 cells 107 / 88 with 16 x 16 x 8 tiles (one launch per colour 143 /
-// 93).  A 64^3 step takes 5.41 ms with 8 x 8 x 8 tiles at 64^3 cells, 5.66 with
-// 16 x 16 x 8.
-constexpr long kMacRegTile = 131072, kMacBigTile = 400000;
-
 template <class T, int NSW, int SRC, bool REST>
-inline void mac_tile_launch(MacTileArgs<T> a, hipStream_t s) {
+inline void mac_tile_launch(MacTileArgs<T> a, const MacTiles& tiles, hipStream_t s) {
     const long n = (long)a.g.n[0] * a.g.n[1] * a.g.n[2];
     a.gz = (a.g.n[2] + 7) / 8;
-    if constexpr (NSW == 2)
-        if (n >= kMacBigTile) {
+    if constexpr (NSW > 0)
+        if (n > tiles.big) {
             a.gx = (a.g.n[0] + 15) / 16;
             a.gy = (a.g.n[1] + 15) / 16;
             mac_tile_kernel<T, 16, 16, 8, NSW, SRC, REST><<<a.gx * a.gy * a.gz, 512, 0, s>>>(a);
@@ -358,8 +350,8 @@ inline void mac_tile_launch(MacTileArgs<T> a, hipStream_t s) {
         }
     a.gx = (a.g.n[0] + 7) / 8;
     a.gy = (a.g.n[1] + 7) / 8;
-    if constexpr (NSW == 2)
-        if (n > kMacRegTile) {
+    if constexpr (NSW > 0)
+        if (n > tiles.reg) {
             mac_tile_kernel<T, 8, 8, 8, NSW, SRC, REST><<<a.gx * a.gy * a.gz, 512, 0, s>>>(a);
             return;
         }
@@ -367,24 +359,32 @@ inline void mac_tile_launch(MacTileArgs<T> a, hipStream_t s) {
 }
 
 template <class T, int NSW>
-inline void mac_tile_leg(const MacTileArgs<T>& a, int src, bool rest, hipStream_t s) {
+inline void mac_tile_leg(const MacTileArgs<T>& a, int src, bool rest, const MacTiles& tiles, hipStream_t s) {
     if (src == MT_ZERO) {
-        if (rest) mac_tile_launch<T, NSW, MT_ZERO, true>(a, s);
-        else mac_tile_launch<T, NSW, MT_ZERO, false>(a, s);
+        if (rest) mac_tile_launch<T, NSW, MT_ZERO, true>(a, tiles, s);
+        else mac_tile_launch<T, NSW, MT_ZERO, false>(a, tiles, s);
     } else if (src == MT_X) {
-        if (rest) mac_tile_launch<T, NSW, MT_X, true>(a, s);
-        else mac_tile_launch<T, NSW, MT_X, false>(a, s);
+        if (rest) mac_tile_launch<T, NSW, MT_X, true>(a, tiles, s);
+        else mac_tile_launch<T, NSW, MT_X, false>(a, tiles, s);
     } else {
-        mac_tile_launch<T, NSW, MT_PROLONG, false>(a, s);
+        mac_tile_launch<T, NSW, MT_PROLONG, false>(a, tiles, s);
     }
 }
 
-// nu sweeps as an odd number of launches of at most 2 sweeps, alternating
-// between xa and xb and ending in xb (the first reads xa unless src is MT_ZERO)
+// Launches of the down and the up leg, at most 2 sweeps each: the fewest with an
+// even sum, after which the iterate is back in the buffer it started from (128^3
+// cells with 3 + 3 sweeps: 2 + 2 launches)
+inline void mac_leg_launches(int nu1, int nu2, int& down, int& up) {
+    down = std::max(1, (nu1 + 1) / 2);
+    up = std::max(1, (nu2 + 1) / 2);
+    if ((down + up) % 2) ++(up > down ? up : down);  // that leg has 3 sweeps or more
+}
+
+// nu sweeps as m launches, alternating between the buffers (the first reads xa
+// unless src is MT_ZERO)
 template <class T>
-inline void mac_tile_sweeps(MacTileArgs<T> a, int src, T* xa, T* xb, int nu, bool rest, hipStream_t s) {
-    int m = std::max(1, (nu + 1) / 2);
-    if (m % 2 == 0) ++m;
+inline void mac_tile_sweeps(MacTileArgs<T> a, int src, T* xa, T* xb, int nu, int m, bool rest,
+                            const MacTiles& tiles, hipStream_t s) {
     for (int q = 0; q < m; ++q) {
         const int sw = std::min(2, nu - (m - 1 - q));  // leave at least one per later launch
         nu -= std::max(sw, 0);
@@ -392,9 +392,9 @@ inline void mac_tile_sweeps(MacTileArgs<T> a, int src, T* xa, T* xb, int nu, boo
         a.xout = q % 2 == 0 ? xb : xa;
         const int from = q == 0 ? src : MT_X;
         const bool r = rest && q == m - 1;
-        if (sw >= 2) mac_tile_leg<T, 2>(a, from, r, s);
-        else if (sw == 1) mac_tile_leg<T, 1>(a, from, r, s);
-        else mac_tile_leg<T, 0>(a, from, r, s);
+        if (sw >= 2) mac_tile_leg<T, 2>(a, from, r, tiles, s);
+        else if (sw == 1) mac_tile_leg<T, 1>(a, from, r, tiles, s);
+        else mac_tile_leg<T, 0>(a, from, r, tiles, s);
     }
 }
 

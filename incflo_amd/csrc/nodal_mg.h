@@ -147,6 +147,15 @@ class TileSet {
 // one-workgroup coarse cycle takes (tuning table mac_coarse_cells; 0: none)
 long mac_coarse_cells();
 
+// Tiles of a cell-centred level's legs by its cells: registers up to reg, 8 x 8 x 8
+// in LDS up to big, 16 x 16 x 8 above; FP32 levels of more than max cells whose rows
+// are whole 128-byte lines: one launch per colour (tuning table mac_tiles)
+struct MacTiles {
+    long reg, big, max;
+    bool operator==(const MacTiles& o) const { return reg == o.reg && big == o.big && max == o.max; }
+};
+MacTiles mac_tiles();
+
 // nodes up to which an embedded-boundary level has all its rows in the table
 // (tuning table eb_row_nodes)
 long eb_row_nodes();

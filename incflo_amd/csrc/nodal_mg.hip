@@ -101,6 +101,22 @@ long eb_row_nodes() {
     return g_eb_row_nodes;
 }
 
+// Legs of the cell-centred V-cycle (mac_tile_kernels.h).
+// Per leg (down / up, FP64): 48 x 32 x 24 cells 11 / 11.6 us with registers, 16 / 13
+// without; 96 x 64 x 48 cells 35 / 35 with, 28 / 23 without (one launch per colour
+// took 49 / 38); 128^3 cells 107 / 88 with 16 x 16 x 8 tiles (one launch per colour 143 /
+// 93).  A 64^3 step takes 5.41 ms with 8 x 8 x 8 tiles at 64^3 cells, 5.66 with
+// 16 x 16 x 8.  In FP32 a colour streams half the bytes, and on large levels eight
+// colours cost less than the halos of two legs: 256^3 cells 98 us per colour, 704 /
+// 480 per leg.
+static const MacTiles kMacTiles{131072, 400000, 8000000};
+static MacTiles g_mac_tiles = kMacTiles;
+
+MacTiles mac_tiles() {
+    std::lock_guard<std::mutex> lk(g_tune_mtx);
+    return g_mac_tiles;
+}
+
 long mac_coarse_cells() {
     std::lock_guard<std::mutex> lk(g_tune_mtx);
     return g_mac_coarse_cells;
@@ -1200,6 +1216,7 @@ std::string tuning_table() {
     o << "amr_tile_width " << g_amr_tile_width << "\n";
     o << "amr_tile_width32 " << g_amr_tile_width32 << "\n";
     o << "amr_tile_kz " << g_amr_tile_kz << "\n";
+    o << "mac_tiles " << g_mac_tiles.reg << " " << g_mac_tiles.big << " " << g_mac_tiles.max << "\n";
     o << "eb_row_nodes " << g_eb_row_nodes << "\n";
     return o.str();
 }
@@ -1209,6 +1226,7 @@ void set_tuning_table(const std::string& text) {
     std::string tag;
     std::map<ShapeKey, StencilShape> shapes;
     long coarse = 1, mac_coarse = 512, eb_rows = 200000;
+    MacTiles mtiles = kMacTiles;
     int pairs = 0, tilew = 16, tilew32 = 64, tilekz = TileSet::kKZ;
     while (in >> tag) {
         if (tag == "stencil") {
@@ -1240,6 +1258,10 @@ void set_tuning_table(const std::string& text) {
         } else if (tag == "mac_coarse_cells") {
             in >> mac_coarse;
             MGX_REQUIRE(!in.fail() && mac_coarse >= 0, MGX_ERR_ARG, "tuning table: bad mac_coarse_cells");
+        } else if (tag == "mac_tiles") {
+            in >> mtiles.reg >> mtiles.big >> mtiles.max;
+            MGX_REQUIRE(!in.fail() && mtiles.reg >= 0 && mtiles.big >= mtiles.reg && mtiles.max >= 0,
+                        MGX_ERR_ARG, "tuning table: bad mac_tiles");
         } else if (tag == "eb_row_nodes") {
             in >> eb_rows;
             MGX_REQUIRE(!in.fail() && eb_rows >= 0, MGX_ERR_ARG, "tuning table: bad eb_row_nodes");
@@ -1256,6 +1278,7 @@ void set_tuning_table(const std::string& text) {
     g_coarse_nodes = coarse;
     g_mac_coarse_cells = mac_coarse;
     g_eb_row_nodes = eb_rows;
+    g_mac_tiles = mtiles;
     g_jacobi_pairs = pairs;
     g_amr_tile_width = tilew;
     g_amr_tile_width32 = tilew32;

@@ -232,6 +232,10 @@ MGX_API int mgx_nodal_autotune(mgx_nodal h, int mode, char* report, int report_l
  * "amr_tile_width32 16|64" (FP32) and "amr_tile_kz K" planes, and
  * "mac_coarse_cells N": cell-centred multigrid levels below the first with
  * at most N cells run in one workgroup per V-cycle half, 0: none;
+ * "mac_tiles REG BIG MAX": cell-centred levels of at most REG cells are smoothed
+ * on register tiles, up to BIG on 8 x 8 x 8 and larger ones on 16 x 16 x 8 tiles
+ * in LDS, FP32 levels of more than MAX cells and rows of a multiple of 32 with one
+ * launch per colour;
  * "eb_row_nodes N": embedded-boundary levels of at most N nodes are swept from
  * assembled rows alone, on handles set up later), for caching
  * per device model; mgx_tuning_set loads such a text (replacing the table;
