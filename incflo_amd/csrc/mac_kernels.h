@@ -43,6 +43,13 @@ __device__ __forceinline__ long fidx(const MGeomK& g, int d, int i, int j, int k
     return i + f0 * (j + f1 * (long)k);
 }
 
+// A cell's update, residual and restriction have the same bits in every kernel
+// that makes them (one launch per colour, tiles of each kind, the one-workgroup
+// coarse cycle): products are fused into an addition only where one expression
+// says so, and the weights are values of their own (formed inside the branches: before them, every one
+// waits for its coefficient and the 256^3 residual takes 253 us instead of 196).
+#pragma clang fp contract(on)
+
 // (L phi)_c and the diagonal of L at cell (i,j,k); phi read with direct loads.
 template <class T, class TB, class TP>
 __device__ __forceinline__ T mac_apply_cell(const MGeomK& g, const MCoef<T>& c, const TB* bx,
@@ -60,11 +67,13 @@ __device__ __forceinline__ T mac_apply_cell(const MGeomK& g, const MCoef<T>& c, 
             const T b = (T)beta[d][fidx(g, d, q[0], q[1], q[2])];
             if (p[d] > 0 || g.per[d]) {
                 q[d] = p[d] > 0 ? p[d] - 1 : g.n[d] - 1;
-                acc += c.ih2[d] * b * ((T)phi[cidx(g, q[0], q[1], q[2])] - pc);
-                dg -= c.ih2[d] * b;
+                const T w = c.ih2[d] * b;
+                acc += w * ((T)phi[cidx(g, q[0], q[1], q[2])] - pc);
+                dg -= w;
             } else if (g.dlo[d]) {
-                acc -= 2 * c.ih2[d] * b * pc;
-                dg -= 2 * c.ih2[d] * b;
+                const T w = 2 * c.ih2[d] * b;
+                acc -= w * pc;
+                dg -= w;
             }
         }
         // hi face
@@ -74,11 +83,13 @@ __device__ __forceinline__ T mac_apply_cell(const MGeomK& g, const MCoef<T>& c, 
             const T b = (T)beta[d][fidx(g, d, q[0], q[1], q[2])];
             if (p[d] + 1 < g.n[d] || g.per[d]) {
                 q[d] = p[d] + 1 < g.n[d] ? p[d] + 1 : 0;
-                acc += c.ih2[d] * b * ((T)phi[cidx(g, q[0], q[1], q[2])] - pc);
-                dg -= c.ih2[d] * b;
+                const T w = c.ih2[d] * b;
+                acc += w * ((T)phi[cidx(g, q[0], q[1], q[2])] - pc);
+                dg -= w;
             } else if (g.dhi[d]) {
-                acc -= 2 * c.ih2[d] * b * pc;
-                dg -= 2 * c.ih2[d] * b;
+                const T w = 2 * c.ih2[d] * b;
+                acc -= w * pc;
+                dg -= w;
             }
         }
     }
@@ -260,6 +271,8 @@ static __global__ void __launch_bounds__(1024) mac_coarse_cycle_kernel(MacCoarse
         }
     }
 }
+
+#pragma clang fp contract(fast)
 
 // coarse face beta = mean of the 4 fine faces covering it
 template <class T, class TF>

@@ -23,6 +23,8 @@
 
 namespace mgx {
 
+#pragma clang fp contract(on)  // as in mac_kernels.h
+
 enum { MT_ZERO = 0, MT_X = 1, MT_PROLONG = 2 };  // x starts from 0, xin, xin + parent's xc
 
 template <class T>
@@ -55,18 +57,22 @@ __device__ __forceinline__ T mac_apply_lds(const MGeomK& g, const MCoef<T>& c, c
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         if (pos[d] > 0 || g.per[d]) {
-            acc += c.ih2[d] * bl[d] * (p[-st[d]] - pc);
-            dg -= c.ih2[d] * bl[d];
+            const T w = c.ih2[d] * bl[d];
+            acc += w * (p[-st[d]] - pc);
+            dg -= w;
         } else if (g.dlo[d]) {
-            acc -= 2 * c.ih2[d] * bl[d] * pc;
-            dg -= 2 * c.ih2[d] * bl[d];
+            const T w = 2 * c.ih2[d] * bl[d];
+            acc -= w * pc;
+            dg -= w;
         }
         if (pos[d] + 1 < g.n[d] || g.per[d]) {
-            acc += c.ih2[d] * bh[d] * (p[st[d]] - pc);
-            dg -= c.ih2[d] * bh[d];
+            const T w = c.ih2[d] * bh[d];
+            acc += w * (p[st[d]] - pc);
+            dg -= w;
         } else if (g.dhi[d]) {
-            acc -= 2 * c.ih2[d] * bh[d] * pc;
-            dg -= 2 * c.ih2[d] * bh[d];
+            const T w = 2 * c.ih2[d] * bh[d];
+            acc -= w * pc;
+            dg -= w;
         }
     }
     if (acoef) {
@@ -261,8 +267,8 @@ static __global__ void __launch_bounds__(512) mac_reg_tile_kernel(MacTileArgs<T>
 #pragma unroll
                 for (int d = 0; d < 3; ++d) {
                     T lo = a.c.ih2[d] * bl[d], hi = a.c.ih2[d] * bh[d];
-                    if (!(p[d] > 0 || g.per[d])) lo = g.dlo[d] ? 2 * a.c.ih2[d] * bl[d] : (T)0;
-                    if (!(p[d] + 1 < g.n[d] || g.per[d])) hi = g.dhi[d] ? 2 * a.c.ih2[d] * bh[d] : (T)0;
+                    if (!(p[d] > 0 || g.per[d])) lo = g.dlo[d] ? 2 * lo : (T)0;
+                    if (!(p[d] + 1 < g.n[d] || g.per[d])) hi = g.dhi[d] ? 2 * hi : (T)0;
                     c.t[2 * d] = lo;
                     c.t[2 * d + 1] = hi;
                     dg -= lo;
@@ -336,6 +342,8 @@ static __global__ void __launch_bounds__(512) mac_reg_tile_kernel(MacTileArgs<T>
         }
     }
 }
+
+#pragma clang fp contract(fast)
 
 template <class T, int NSW, int SRC, bool REST>
 inline void mac_tile_launch(MacTileArgs<T> a, const MacTiles& tiles, hipStream_t s) {
