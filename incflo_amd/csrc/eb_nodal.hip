@@ -362,29 +362,26 @@ void row_nodes(EBLevelData& lv) {
     lv.all_rows = nn <= eb_row_nodes();
     lv.nrow = (int)nn;
     if (!lv.all_rows) {
+        // the active nodes of cells that are not regular, from those cells
         std::vector<unsigned char> type(lv.mask_h);
-        std::vector<int> ids;
-        for (int k = 0; k < g.nn[2]; ++k)
-            for (int j = 0; j < g.nn[1]; ++j)
-                for (int i = 0; i < g.nn[0]; ++i) {
-                    const int id = i + g.nn[0] * (j + g.nn[1] * k);
-                    if (!type[id]) continue;
-                    const int n3[3] = {i, j, k};
-                    bool plain = true;
-                    for (int a = 0; a < 8 && plain; ++a) {
-                        int c[3];
-                        bool in = true;
+        for (int k = 0; k < g.n[2]; ++k)
+            for (int j = 0; j < g.n[1]; ++j)
+                for (int i = 0; i < g.n[0]; ++i) {
+                    if (lv.cidx_h[i + (long)g.n[0] * (j + (long)g.n[1] * k)] == -1) continue;
+                    const int c[3] = {i, j, k};
+                    for (int a = 0; a < 8; ++a) {
+                        int m[3];
                         for (int d = 0; d < 3; ++d) {
-                            c[d] = n3[d] - 1 + ((a >> d) & 1);
-                            if (g.per[d]) c[d] = (c[d] + g.n[d]) % g.n[d];
-                            else in = in && c[d] >= 0 && c[d] < g.n[d];
+                            m[d] = c[d] + ((a >> d) & 1);
+                            if (m[d] == g.nn[d]) m[d] = 0;  // periodic: the image of node 0
                         }
-                        plain = !in || lv.cidx_h[c[0] + (long)g.n[0] * (c[1] + (long)g.n[1] * c[2])] == -1;
+                        unsigned char& t = type[m[0] + (long)g.nn[0] * (m[1] + (long)g.nn[1] * m[2])];
+                        if (t == 1) t = 2;
                     }
-                    if (plain) continue;
-                    type[id] = 2;
-                    ids.push_back(id);
                 }
+        std::vector<int> ids;
+        for (long id = 0; id < nn; ++id)
+            if (type[id] == 2) ids.push_back((int)id);
         lv.nrow = (int)ids.size();
         upload(lv.ids, ids);
         upload(lv.types, type);
