@@ -193,7 +193,7 @@ struct LevelChoice {
         }
         if (n == 0) first = prev;
         n += ran;
-        if (deep && !(rn < 2.0 * first)) {
+        if (deep && !(rn < 10.0 * first)) {
             rho[1] = HUGE_VAL;
             deep = false;
             n = 0;
