@@ -24,7 +24,7 @@
 // with its vectors and index divisions in LDS or global memory before it:
 //   nodal 1280 nodes (120 x 72 x 56 channel)          592 -> 150 us
 //   nodal 2275 nodes (256 x 16 x 24 channel)         2370 -> 527 us
-//   nodal 10440 nodes (224 x 232 x 88 channel)       6730 -> 3680 us
+//   nodal 10440 nodes (224 x 232 x 88 channel)       5280 -> 3570 us
 //   EB nodal 425 nodes (256 x 64 x 64 channel)       1130 -> 70 us
 //   MAC 480 cells (160 x 24 x 16 channel at 2 levels) 1320 -> 200 us
 #pragma once
